@@ -208,8 +208,15 @@ def path_ms(t):
 def gemm_instance(m, n, k, bm, epi, cus):
     """The kernel instance the engine launches for an m x n x k GEMM with tile height bm (one
     K split)."""
-    if bm >= 128:
-        return f"gemm_big<{bm}, {jh.EPI[epi]}, false>"
+    if bm >= 128:  # the throughput kernel the launch takes (gemm_pick in csrc/gemm.hip)
+        ks, ceil = k / 768, lambda a, b: -(-a // b)
+        l128 = ceil(n // 128 * ceil(m, 128), cus)
+        c128 = 2 + 8.5 * ks if l128 == 1 else 2.5 + 7.6 * ks * l128
+        rounds = lambda h: ceil(n // 256 * ceil(m, h), cus)
+        h = min((256, 224, 192, 160), key=lambda h: rounds(h) * (h + 53))
+        if n % 256 == 0 and 4.5 + rounds(h) * (0.2 + h / 80 + ks * (3.2 + h / 20)) < c128:
+            return f"gemm_wide<{h}, {jh.EPI[epi]}, false>"
+        return f"gemm_big<{jh.EPI[epi]}, false>"
     if (n // 64) * -(-m // bm) <= cus and k >= 256:  # the eight-wave instance: a block a CU at most
         most = (k // 32 + 7) // 8  # K steps of the busiest wave: its K path
         path = 3 if most <= 3 else 5 if most <= 5 else 6 if most <= 6 and bm <= 32 else 1

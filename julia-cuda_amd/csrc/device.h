@@ -229,6 +229,20 @@ __device__ __forceinline__ half8 bload16(__amdgpu_buffer_rsrc_t r, uint32_t byte
     return __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, XG ? 16 : 0));
 }
 
+__device__ __forceinline__ float bload4(__amdgpu_buffer_rsrc_t r, uint32_t byte_off) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, byte_off, 0, 0));
+}
+template <bool XG>
+__device__ __forceinline__ float2 bload8(__amdgpu_buffer_rsrc_t r, uint32_t byte_off) {
+    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, byte_off, 0, XG ? 16 : 0));
+}
+
+// 8-byte buffer store, device-coherent.
+__device__ __forceinline__ void bstore8(__amdgpu_buffer_rsrc_t r, uint32_t byte_off, float2 v) {
+    typedef int int2_t __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(int2_t, v), r, byte_off, 0, 16);
+}
+
 // 16-byte buffer store at byte_off; with XG device-coherent (sc1) in one instruction, where a
 // coherent global store takes two 8-byte ones.
 template <bool XG>

@@ -149,7 +149,7 @@ struct Engine {
         g.epi = epi, g.a = a, g.w = w, g.c = c, g.m = m, g.n = n, g.k = k;
         g.stats_in = stats_in, g.colsum = colsum, g.eps = eps, g.bias = bias;
         g.rope = rope, g.pos = pos, g.rope_rows = cfg.max_positions, g.stats_out = stats_out;
-        gemm_launch(g, gemm_choose(m, n, k, cus, epi), scratch, stream);
+        gemm_launch(g, gemm_pick(m, n, k, cus, epi), scratch, stream);
     }
 
     // Layer l's five steps as five launches (src/forward.rs:105-165, 361-424): qkv (RoPE; the
@@ -326,9 +326,9 @@ struct Engine {
         // epilogue (EPI_SCORE), where the chooser gives those GEMMs latency tiles (lin1 without
         // a K split); otherwise a gather kernel and a score kernel run.
         auto lat = [&](GemmConfig c) { return c.bm < 128; };
-        const GemmConfig cs = compact ? gemm_choose(nm, d, d, cus, EPI_K_LNBIASGELU) : GemmConfig{};
+        const GemmConfig cs = compact ? gemm_pick(nm, d, d, cus, EPI_K_LNBIASGELU) : GemmConfig{};
         const bool fold = compact && lat(cs) && cs.splits == 1 &&
-                          (L == 0 || lat(gemm_choose(nm, d, d, cus, EPI_K_BIASRESSTATS)));
+                          (L == 0 || lat(gemm_pick(nm, d, d, cus, EPI_K_BIASRESSTATS)));
         // The marker rows' residual stream: x is free once norm_add has read the encoder's
         // output; their attention output goes to qkv (free once attention has read it).
         jh_half* hr = hx;
@@ -348,7 +348,7 @@ struct Engine {
                 g.epi = EPI_K_BIASRESSTATS | EPI_GATHER, g.a = o, g.w = h(H.out_proj), g.c = x;
                 g.m = nm, g.n = d, g.k = d, g.bias = f(H.out_proj_b), g.stats_out = stats_b;
                 g.res = hx, g.rows = markers, g.src_m = n;
-                gemm_launch(g, gemm_choose(nm, d, d, cus, g.epi), scratch, stream);
+                gemm_launch(g, gemm_pick(nm, d, d, cus, g.epi), scratch, stream);
                 hr = x, m = nm;
             } else {
                 const jh_half* ao = o;
@@ -500,7 +500,7 @@ Engine* load_engine(const char* dir, size_t max_length, size_t batch_rows = 0) {
                              {c.head_ff, (int)d, EPI_LN},   {(int)d, c.head_ff, 0}};
     for (int m = 1; m <= (int)n; m++) {
         for (auto& s : shapes) {
-            const GemmConfig cfg = gemm_choose(m, s[0], s[1], e->cus, s[2]);
+            const GemmConfig cfg = gemm_pick(m, s[0], s[1], e->cus, s[2]);
             ws = std::max(ws, gemm_ws_floats(m, s[0], cfg));
             counters = std::max(counters, gemm_counters(m, s[0], cfg));
         }
@@ -840,7 +840,7 @@ int julia_hip_gemm(const julia_hip_gemm_args* g, julia_hip_gemm_config cfg,
     return guarded(err, err_len, [&] {
         const Gemm x = to_gemm(g);
         GemmConfig c{cfg.bm, cfg.splits};
-        if (c.bm == 0) c = gemm_choose(x.m, x.n, x.k, device_cus(), x.epi);
+        if (c.bm == 0) c = gemm_pick(x.m, x.n, x.k, device_cus(), x.epi);
         gemm_launch(x, c, scratch_of(s), (hipStream_t)stream);
     });
 }
@@ -850,7 +850,7 @@ int julia_hip_gemm_static(const julia_hip_gemm_args* g, julia_hip_gemm_config cf
     return guarded(err, err_len, [&] {
         const Gemm x = to_gemm(g);
         GemmConfig c{cfg.bm, cfg.splits};
-        if (c.bm == 0) c = gemm_choose(x.m, x.n, x.k, device_cus(), x.epi);
+        if (c.bm == 0) c = gemm_pick(x.m, x.n, x.k, device_cus(), x.epi);
         gemm_launch_static(x, c, (hipStream_t)stream);
     });
 }
@@ -906,7 +906,7 @@ int julia_hip_time_gemm(const julia_hip_gemm_args* g, julia_hip_gemm_config cfg,
     return guarded(err, err_len, [&] {
         const Gemm x = to_gemm(g);
         GemmConfig c{cfg.bm, cfg.splits};
-        if (c.bm == 0) c = gemm_choose(x.m, x.n, x.k, device_cus(), x.epi);
+        if (c.bm == 0) c = gemm_pick(x.m, x.n, x.k, device_cus(), x.epi);
         const Scratch sc = scratch_of(s);
         gemm_check(x, c, sc);
         hipStream_t st = nullptr;
@@ -1195,7 +1195,7 @@ int julia_hip_time_encoder_step(const Engine* ce, int step, int m, int bm, int s
         hip_check(hipStreamSynchronize(e.stream), "time");
         int l = 0;
         auto gemm_cfg = [&](int n, int k, int epi) {
-            return bm > 0 ? GemmConfig{bm, splits} : gemm_choose(m, n, k, e.cus, epi);
+            return bm > 0 ? GemmConfig{bm, splits} : gemm_pick(m, n, k, e.cus, epi);
         };
         // Rotate through the layers' weights, as the reference's --time does (src/main.rs:
         // 307-312), so the weights are not the last call's, still in L2. Layer 0 has no

@@ -12,12 +12,14 @@
 //    gemm_lat runs four waves streaming a and w fragments from L2 into registers, two blocks a
 //    CU. Grid split-K on top is deterministic: the last block of a tile to arrive sums every
 //    split's partial in split order.
-//  - gemm_big (128 x 128, 192 x 256 or 256 x 256 tiles): the MFMA-bound regime (M >= 2048): a
-//    and w tiles copied into four LDS stages by direct buffer -> LDS loads (gemm_big.h), four or
-//    eight waves each owning a 64 x 64 (96 x 64, 128 x 64) output block on 32 x 32 x 16 MFMA, the
-//    epilogue's column-wise part applied on the accumulators. A K split, the same deterministic
-//    last-arriver sum, is there for completeness (config sweeps): at these sizes the chooser
-//    never picks one.
+//  - gemm_big (128 x 128 tiles): the middle sizes and widths that 256 does not divide: a and w
+//    tiles copied into four LDS stages by direct buffer -> LDS loads (gemm_big.h), four waves each
+//    owning a 64 x 64 output block on 32 x 32 x 16 MFMA, the epilogue's column-wise part applied on
+//    the accumulators.
+//  - gemm_wide (160 to 256 rows x 256 columns, gemm_wide.h): the MFMA-bound regime: eight waves on
+//    16 x 16 x 32 MFMA, 64-wide stages, one stream of stage copies over a block's tasks.
+// A K split of the throughput tiles, the same deterministic last-arriver sum, is there for
+// completeness (config sweeps): at these sizes the chooser never picks one.
 //
 // Both apply the epilogues of device.h (LayerNorm folding, bias, ReLU/GELU, RoPE, GeGLU,
 // residual, output statistics) in the same order.
@@ -28,6 +30,7 @@
 
 #include "gemm_big.h"
 #include "gemm_tile.h"
+#include "gemm_wide.h"
 
 namespace jh {
 
@@ -56,19 +59,17 @@ __global__ __launch_bounds__(512, 1) void gemm_lat1(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// gemm_big: BM x BM tiles (BM = 128 or 256) for large M; see gemm_big.h. Dynamic LDS:
-// Big<BM, BM>::LDS_BYTES.
-// Persistent: the grid is the resident blocks (one 256 x 256 or two 128 x 128 a CU), and block
-// b takes tasks b, b + grid, ...: a CU goes from one tile's epilogue to the next tile's copies
-// without a block dispatch in between. (The grid is a multiple of 8, so a block's tasks stay on
-// its XCD's range of xcd_task.)
+// gemm_big: 128 x 128 tiles; see gemm_big.h. Dynamic LDS: Big::LDS_BYTES.
+// Persistent: the grid is the resident blocks (two a CU), and block b takes tasks b, b + grid, ...:
+// a CU goes from one tile's epilogue to the next tile's copies without a block dispatch in
+// between. (The grid is a multiple of 8, so a block's tasks stay on its XCD's range of xcd_task.)
 // SPLIT: K split p.splits ways, the tile's last arriving split running the epilogue.
-template <int BM, int EPI, bool SPLIT>
-__global__ __launch_bounds__((Big<BM, big_bn(BM)>::THREADS)) void gemm_big(GemmParams p) {
+template <int EPI, bool SPLIT>
+__global__ __launch_bounds__(Big::THREADS) void gemm_big(GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) char lds_dyn[];
     const int T = p.tiles_n * p.tiles_m * (SPLIT ? p.splits : 1);
     for (int task = blockIdx.x; task < T; task += gridDim.x)  // each task ends with a block barrier
-        gemm_big_tile<BM, big_bn(BM), EPI, false, false, SPLIT>(p, task, lds_dyn);
+        gemm_big_tile<EPI, false, false, SPLIT>(p, task, lds_dyn);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -128,9 +129,9 @@ void gemm_check(const Gemm& g, GemmConfig cfg, const Scratch& s) {
         fail("no tile height " + std::to_string(cfg.bm));
     if (tput && g.n % big_bn(cfg.bm))
         fail("the " + cfg_str(cfg) + " tiles need n % " + std::to_string(big_bn(cfg.bm)) + " == 0");
-    if (tput && (g.epi & EPI_LN) && g.k > 128 * BIG_LN_SLOTS)
+    if (tput && (g.epi & EPI_LN) && g.k > GEMM_BIG_LN_MAX_K)
         fail("the " + cfg_str(cfg) + " tiles take LayerNorm epilogues up to k = " +
-             std::to_string(128 * BIG_LN_SLOTS));
+             std::to_string(GEMM_BIG_LN_MAX_K));
     const int ksteps = g.k / 32;
     if (cfg.splits < 1 || cfg.splits > 8 || cfg.splits > ksteps)
         fail(std::to_string(cfg.splits) + " splits for " + std::to_string(ksteps) + " K steps");
@@ -187,16 +188,15 @@ void gemm_check(const Gemm& g, GemmConfig cfg, const Scratch& s) {
              std::to_string(ksteps));
 }
 
-template <int B, int EPI, bool SPLIT>
+template <int EPI, bool SPLIT>
 static void launch_big(const GemmParams& p, hipStream_t st) {
-    using C = Big<B, big_bn(B)>;
     static const bool lds_ok =  // once per instantiation, before its first launch
-        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_big<B, EPI, SPLIT>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES) == hipSuccess;
+        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_big<EPI, SPLIT>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, Big::LDS_BYTES) == hipSuccess;
     if (!lds_ok) throw std::runtime_error("gemm: the throughput kernel cannot have its LDS");
     const int blocks = p.tiles_n * p.tiles_m * p.splits;
-    const int grid = std::min(blocks, (B == 128 ? 2 : 1) * device_cus());
-    hipLaunchKernelGGL((gemm_big<B, EPI, SPLIT>), dim3(grid), dim3(C::THREADS), (C::LDS_BYTES), st, p);
+    const int grid = std::min(blocks, 2 * device_cus());
+    hipLaunchKernelGGL((gemm_big<EPI, SPLIT>), dim3(grid), dim3(Big::THREADS), (Big::LDS_BYTES), st, p);
 }
 
 template <int BM, int EPI, int KP>
@@ -235,17 +235,6 @@ static void launch_lat(const GemmParams& p, hipStream_t st) {
     }
 }
 
-template <int BM, int EPI>
-static void launch_one(const GemmParams& p, hipStream_t st) {
-    if (BM >= 128) {
-        constexpr int B = BM >= 128 ? BM : 128;
-        if (p.splits > 1) launch_big<B, EPI, true>(p, st);
-        else launch_big<B, EPI, false>(p, st);
-    } else {
-        launch_lat<BM < 128 ? BM : 64, EPI>(p, st);
-    }
-}
-
 // The epilogues only the latency tiles take (the score, gathered rows).
 template <int EPI>
 static void launch_epi_lat(const GemmParams& p, int bm, hipStream_t st) {
@@ -259,15 +248,10 @@ static void launch_epi_lat(const GemmParams& p, int bm, hipStream_t st) {
 
 template <int EPI>
 static void launch_epi(const GemmParams& p, int bm, hipStream_t st) {
-    switch (bm) {
-        case 16: launch_one<16, EPI>(p, st); break;
-        case 32: launch_one<32, EPI>(p, st); break;
-        case 48: launch_one<48, EPI>(p, st); break;
-        case 64: launch_one<64, EPI>(p, st); break;
-        case 128: launch_one<128, EPI>(p, st); break;
-        case 192: launch_one<192, EPI>(p, st); break;
-        default: launch_one<256, EPI>(p, st); break;
-    }
+    if (bm < 128) return launch_epi_lat<EPI>(p, bm, st);
+    if (bm > 128) return gemm_wide_launch(p, EPI, bm, st);
+    if (p.splits > 1) launch_big<EPI, true>(p, st);
+    else launch_big<EPI, false>(p, st);
 }
 
 void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t st) {
@@ -283,24 +267,25 @@ void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t st
     p.rope_rows = g.rope_rows;
     p.splits = cfg.splits;
     p.tiles_n = g.n / (cfg.bm >= 128 ? big_bn(cfg.bm) : 64);
-    p.tiles_m = (g.m + cfg.bm - 1) / cfg.bm;
+    const int bm = cfg.height ? cfg.height : cfg.bm;
+    p.tiles_m = (g.m + bm - 1) / bm;
     switch (g.epi) {
-        case EPI_K_ROPE: launch_epi<EPI_K_ROPE>(p, cfg.bm, st); break;
-        case EPI_K_LNROPE: launch_epi<EPI_K_LNROPE>(p, cfg.bm, st); break;
-        case EPI_K_LNGEGLU: launch_epi<EPI_K_LNGEGLU>(p, cfg.bm, st); break;
-        case EPI_K_RESSTATS: launch_epi<EPI_K_RESSTATS>(p, cfg.bm, st); break;
-        case EPI_K_LNBIAS: launch_epi<EPI_K_LNBIAS>(p, cfg.bm, st); break;
-        case EPI_K_LNBIASRELU: launch_epi<EPI_K_LNBIASRELU>(p, cfg.bm, st); break;
-        case EPI_K_LNBIASGELU: launch_epi<EPI_K_LNBIASGELU>(p, cfg.bm, st); break;
-        case EPI_K_BIASRESSTATS: launch_epi<EPI_K_BIASRESSTATS>(p, cfg.bm, st); break;
+        case EPI_K_ROPE: launch_epi<EPI_K_ROPE>(p, bm, st); break;
+        case EPI_K_LNROPE: launch_epi<EPI_K_LNROPE>(p, bm, st); break;
+        case EPI_K_LNGEGLU: launch_epi<EPI_K_LNGEGLU>(p, bm, st); break;
+        case EPI_K_RESSTATS: launch_epi<EPI_K_RESSTATS>(p, bm, st); break;
+        case EPI_K_LNBIAS: launch_epi<EPI_K_LNBIAS>(p, bm, st); break;
+        case EPI_K_LNBIASRELU: launch_epi<EPI_K_LNBIASRELU>(p, bm, st); break;
+        case EPI_K_LNBIASGELU: launch_epi<EPI_K_LNBIASGELU>(p, bm, st); break;
+        case EPI_K_BIASRESSTATS: launch_epi<EPI_K_BIASRESSTATS>(p, bm, st); break;
         case EPI_K_BIASRESSTATS | EPI_GATHER:
-            launch_epi_lat<EPI_K_BIASRESSTATS | EPI_GATHER>(p, cfg.bm, st);
+            launch_epi_lat<EPI_K_BIASRESSTATS | EPI_GATHER>(p, bm, st);
             break;
-        case EPI_K_LNBIASGELU_SCORE: launch_epi_lat<EPI_K_LNBIASGELU_SCORE>(p, cfg.bm, st); break;
+        case EPI_K_LNBIASGELU_SCORE: launch_epi_lat<EPI_K_LNBIASGELU_SCORE>(p, bm, st); break;
         case EPI_K_LNBIASGELU_SCORE | EPI_GATHER:
-            launch_epi_lat<EPI_K_LNBIASGELU_SCORE | EPI_GATHER>(p, cfg.bm, st);
+            launch_epi_lat<EPI_K_LNBIASGELU_SCORE | EPI_GATHER>(p, bm, st);
             break;
-        case 0: launch_epi<0>(p, cfg.bm, st); break;
+        case 0: launch_epi<0>(p, bm, st); break;
         default: throw std::runtime_error("gemm: no kernel for epilogue " + std::to_string(g.epi));
     }
     const hipError_t e = hipGetLastError();
@@ -379,8 +364,8 @@ void gemm_launch_static(const Gemm& g, GemmConfig cfg, hipStream_t st) {
     gemm_launch(g, cfg, s, st);
 }
 
-// The tiling for a GEMM on a 256-CU GPU: the cheapest of the latency tiles and the three
-// throughput tiles under a cost model fitted to MI355X sweeps (M = 72 .. 18752, the encoder's
+// The tiling for a GEMM on a 256-CU GPU, by name (julia_hip_gemm_choose): the cheapest of the
+// latency tiles and the three throughput tiles under a cost model fitted to MI355X sweeps (M = 72 .. 18752, the encoder's
 // four shapes; microseconds, random operands, weights rotating through the layers).
 //  - Latency tiles (BM = 16/32/48/64 x 64): bound by how fast a CU takes in its tiles'
 //    operands: a fixed ~4 us (launch, first round trip, reduction, epilogue) plus the busiest
@@ -401,7 +386,8 @@ void gemm_launch_static(const Gemm& g, GemmConfig cfg, hipStream_t st) {
 // 192 x 256 for qkv and wi at 4096; 256 x 256 at 6144 and 12288 (qkv, wi) and everything at
 // 18752.
 GemmConfig gemm_choose(int m, int n, int k, int cus, int epi) {
-    static_assert(GEMM_BIG_LN_MAX_K == 128 * BIG_LN_SLOTS, "the LayerNorm limit of the throughput tiles");
+    static_assert(GEMM_BIG_LN_MAX_K == 128 * BIG_LN_SLOTS && GEMM_BIG_LN_MAX_K == 128 * WIDE_LN_SLOTS,
+                  "the LayerNorm limit of the throughput tiles");
     if (cus <= 0) cus = 256;
     GemmConfig best{32, 1};
     double best_cost = 1e30;
@@ -424,6 +410,33 @@ GemmConfig gemm_choose(int m, int n, int k, int cus, int epi) {
             const double c192 = 2.0 + 21.7 * ks * (double)l192;
             if (c192 < best_cost) best_cost = c192, best = GemmConfig{192, 1};
         }
+    }
+    return best;
+}
+
+// What a GEMM is run with: gemm_choose's pick, a throughput one decided between the 128 x 128 and the
+// wide tiles at their best height by a model of the kernels as they are (MI355X, random operands):
+//  - 128 x 128 tiles (two a CU): ~2 us plus ~8.5 us (K = 768) for one a CU, ~2.5 us plus 7.6 us
+//    each for more (measured 10.7 us for one, 15-17.5 for two, 25 for three, 39 for five).
+//  - The wide tiles (one a CU): ~4.5 us plus, per round of tiles, the K loop (3.2 + h / 20 us at K =
+//    768, h the tile's rows) and the epilogue (0.2 + h / 80): measured at 160 rows 18.5 us for one
+//    round (4096 x 2304), 33.7 for two (8192), at 224 rows 66 for three (18752).
+// So 128 x 128 for qkv and wi up to ~3000 rows and for wo up to 8192 (17.5 us there against 18.5
+// for the wide tiles; wo_mlp level, 23.5), the wide tiles for qkv and wi from 4096 (18.5 us
+// against 25) and for everything at 18752.
+GemmConfig gemm_pick(int m, int n, int k, int cus, int epi) {
+    GemmConfig best = gemm_choose(m, n, k, cus, epi);
+    if (best.bm < 128) return best;
+    if (cus <= 0) cus = 256;
+    const double ks = (double)k / 768.0;
+    const long l128 = ((long)(n / 128) * ((m + 127) / 128) + cus - 1) / cus;
+    best = GemmConfig{128, 1};
+    if (n % WIDE_BN == 0) {
+        const int h = wide_height(m, n, cus);
+        const long rounds = ((long)(n / WIDE_BN) * ((m + h - 1) / h) + cus - 1) / cus;
+        const double c128 = l128 == 1 ? 2.0 + 8.5 * ks : 2.5 + 7.6 * ks * (double)l128;
+        if (4.5 + (double)rounds * (0.2 + h / 80.0 + ks * (3.2 + h / 20.0)) < c128)
+            best = GemmConfig{256, 1, h};
     }
     return best;
 }

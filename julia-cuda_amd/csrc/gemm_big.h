@@ -1,57 +1,50 @@
-// One output tile of the throughput GEMM (BM x BN = 256 x 256 or 128 x 128), as a device function:
-// the body of the per-GEMM `gemm_big` kernel for large M. c = epilogue(a . w^T) with the
-// epilogues of the latency tile (device.h), applied straight from the accumulators.
+// One 128 x 128 output tile of the throughput GEMM, as a device function: the body of the
+// per-GEMM `gemm_big` kernel for the middle sizes (and widths that the wide tiles' 256 columns do
+// not divide) and a task of the persistent kernel's. c = epilogue(a . w^T) with the epilogues of
+// the latency tile (device.h), applied straight from the accumulators.
 //
-// Waves in a 2 x (BN / 64) grid (eight for 256 x 256: two a SIMD, so that one wave's MFMAs run
-// while the other waits on its copies or LDS reads) each own a (BM / 2) x 64 block of outputs,
-// computed with MFMA 32 x 32 x 16 as MR = BM / 64 row fragments x 2 column fragments, w as the
-// MFMA's A operand: lane l of fragment (i, c) holds output row 32 i + l % 32 and columns
-// 32 c + 8 q + 4 (l / 32) + e, q, e < 4. A 256 x 256 tile reads 64 bytes of operands per
-// 8 Kflop, half what a 256 x 128 tile reads: the copy path into a CU (about 64 bytes per clock)
-// keeps up with the MFMAs.
+// Waves in a 2 x 2 grid each own a 64 x 64 block of outputs, computed with MFMA 32 x 32 x 16 as
+// MR = 2 row fragments x 2 column fragments, w as the MFMA's A operand: lane l of fragment (i, c)
+// holds output row 32 i + l % 32 and columns 32 c + 8 q + 4 (l / 32) + e, q, e < 4. Two tiles a CU
+// where there are as many.
 //
 // The K loop runs BK = 32 at a time through four LDS stages filled by direct buffer -> LDS loads
-// (no register staging), three stages ahead, with one block barrier per stage. A stage's copies
-// are issued between the MFMAs of the stage three back: issued in one burst they stall the
-// issuing wave on the address path while its MFMA unit idles.
-//  - a's stage: BM rows x 64 bytes; copy I takes rows 16 I .. 16 I + 15 (4 lanes a row), lane l
+// (no register staging), three stages ahead, with one block barrier per stage: where a tile has
+// its CU to itself (wo at 4096 rows), the two 64-wide stages of the wide tiles leave its copies'
+// latency bare (10.7 us here, 13.5 so, 11.4 with four of them). A stage's copies are issued between
+// the MFMAs of the stage three back: issued in one burst they stall the issuing wave on the address
+// path while its MFMA unit idles.
+//  - a's stage: 128 rows x 64 bytes; copy I takes rows 16 I .. 16 I + 15 (4 lanes a row), lane l
 //    into LDS chunk 64 I + l, which is row r = 16 I + l / 4, chunk l % 4, and holds a's chunk
 //    (l % 4) ^ ((r / 4) % 4) of that row: the 16 rows one fragment read serves per LDS cycle
 //    cover all 64 banks.
-//  - w's stage: BN / 64 blocks of the fragment-ordered matrix (64 columns x one 32-wide K unit,
+//  - w's stage: 2 blocks of the fragment-ordered matrix (64 columns x one 32-wide K unit,
 //    4 KB contiguous each), copied as they are.
 //
 // The epilogue's column-wise part runs on the accumulators: a lane has MR output rows, so the row
 // data (LayerNorm statistics, positions) is a few values a lane, loaded with the first stage, and
 // each row's mean and rstd are computed once a tile (two threads a row) into LDS; the column
-// data (colsum, bias) is loaded with the first stage into LDS; the rotate-half pair (x, x + 32) of a head and the GeGLU (input, gate) pair sit in one
-// lane. The result goes through LDS into row-contiguous 16-byte pieces for the residual, the
-// output statistics and the stores. The RoPE table rows and the residual are loaded two row
-// fragments ahead, the first two right after the last MFMAs are issued.
+// data (colsum, bias) is loaded with the first stage into LDS; the rotate-half pair (x, x + 32) of a
+// head and the GeGLU (input, gate) pair sit in one lane. The result goes through LDS into
+// row-contiguous 16-byte pieces for the residual, the output statistics and the stores. The RoPE
+// table rows and the residual are loaded two row fragments ahead, the first two right after the last
+// MFMAs are issued.
 #pragma once
 
 #include "gemm_tile.h"
 
 namespace jh {
 
-template <int BM, int BN>
 struct Big {
-    static_assert((BM == 256 && BN == 256) || (BM == 192 && BN == 256) || (BM == 128 && BN == 128),
-                  "tile shape");
-    static constexpr int TM = BM, TN = BN, BK = 32, NSTAGE = 4;
-    static constexpr int WAVES_M = 2, WAVES_N = BN / 64;  // 2 x 4 waves (BN 256) or 2 x 2 (128)
+    static constexpr int BM = 128, BN = 128, BK = 32, NSTAGE = 4;
+    static constexpr int WAVES_M = 2, WAVES_N = BN / 64;
     static constexpr int NWAVES = WAVES_M * WAVES_N, THREADS = 64 * NWAVES;
     static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;  // a wave's block
     static constexpr int MR = WM / 32, NC = WN / 32;  // its 32 x 32 fragments
     static constexpr int NG = WN / 64;                // its 64-column groups
     static constexpr int A_BYTES = BM * BK * 2, W_BYTES = BN * BK * 2;
     static constexpr int STAGE = A_BYTES + W_BYTES;   // bytes per stage
-    static constexpr int NCOPY = STAGE / 1024, A_COPIES = A_BYTES / 1024;  // 1 KB copies a stage
-    // Copies per wave and stage: LOADS for waves below FULL, LOADS - 1 for the rest (192 x 256:
-    // 28 copies over eight waves; the square tiles: LOADS for every wave).
-    static constexpr int LOADS = (NCOPY + NWAVES - 1) / NWAVES;
-    static constexpr int FULL = NCOPY - (LOADS - 1) * NWAVES;
-    static constexpr bool EVEN = FULL == NWAVES && A_BYTES == W_BYTES;
+    static constexpr int LOADS = STAGE / 1024 / NWAVES;  // 1 KB copies a wave and stage: half a's, half w's
     static constexpr int COLS = NSTAGE * STAGE;       // per wave: colsum, bias of its columns
     static constexpr int ROWS = COLS + NWAVES * 2 * WN * 4;  // per row: LayerNorm mean, rstd
     static constexpr int POSR = ROWS + BM * 8;                // per row: RoPE position
@@ -63,7 +56,7 @@ struct Big {
     static_assert(THREADS >= 2 * BM, "two threads a row for the row statistics");
 };
 
-// The column width of the throughput tile BM rows high.
+// The column width of the throughput tile of height bm (GemmConfig): 128 here, the wide tiles' 256.
 __host__ __device__ constexpr int big_bn(int bm) { return bm == 192 ? 256 : bm; }
 
 // LayerNorm statistics slots one thread reads (two threads split a row's K / 64 slots): the big
@@ -79,14 +72,15 @@ constexpr int BIG_LN_SLOTS = 8;
 // 18752). The residual is read through the caches.
 // SPLIT: p.splits K splits a tile (the instances without it keep the whole K loop's code as it
 // is).
-template <int BM, int BN, int EPI, bool AX, bool XG, bool SPLIT = false>
+template <int EPI, bool AX, bool XG, bool SPLIT = false>
 __device__ __forceinline__ void gemm_big_tile(const GemmParams& p, int task, char* lds,
                                               uint64_t* sub = nullptr) {
     auto mark = [&](int i) {  // profiling: thread 0's view of the task's stages
         if (sub && threadIdx.x == 0) sub[i] = wall_clock64();
     };
     mark(0);
-    using C = Big<BM, BN>;
+    using C = Big;
+    constexpr int BM = C::BM, BN = C::BN;
     constexpr int MR = C::MR, NC = C::NC, NG = C::NG;
     // A task is (tile, K split z): the splits of a tile are consecutive tasks, on one XCD.
     const int S = SPLIT ? p.splits : 1;
@@ -145,22 +139,18 @@ __device__ __forceinline__ void gemm_big_tile(const GemmParams& p, int task, cha
     // Stage copies: copy q of the wave's LOADS is load I = w + NWAVES q of the stage's A_BYTES / 1024
     // a loads then W_BYTES / 1024 w loads.
     // (Copies q < LOADS / 2 are a's, the rest w's: the test is on the unrolled q, no branch.)
-    // (The square tiles: copies q < LOADS / 2 are a's, the rest w's, a test on the unrolled q;
-    // 192 x 256: copy I is a's while I < A_COPIES, a wave-uniform test, and copies past NCOPY
-    // are none.)
-    static_assert(!C::EVEN || C::LOADS % 2 == 0, "half the copies a's");
+    static_assert(C::LOADS % 2 == 0 && C::A_BYTES == C::W_BYTES, "half the copies a's");
     // The copies go through buffer descriptors over a and w (the host checks both fit 4 GB): a
     // lane's 32-bit offset of copy q at unit 0, computed once; unit kt adds kt * 64 bytes (a) or
     // kt * 4 KB (w) as the scalar offset. (Global copies take a 64-bit lane address and an added
-    // 64-bit operation a copy: the GEMMs ran 2-6% slower with them.) Copies q past a 192-row
-    // tile's NCOPY get an offset that is never used.
+    // 64-bit operation a copy: the GEMMs ran 2-6% slower with them.)
     const auto abuf = buffer_rsrc(p.a, (uint32_t)min((size_t)p.m * p.k * 2, (size_t)0xFFFFFFFFu));
     const auto wbuf = buffer_rsrc(p.w, (uint32_t)min((size_t)p.n * p.k * 2, (size_t)0xFFFFFFFFu));
     uint32_t coff[C::LOADS];
 #pragma unroll
     for (int q = 0; q < C::LOADS; q++) {
         const int I = w + C::NWAVES * q;
-        if (C::EVEN ? q < C::LOADS / 2 : I < C::A_COPIES) {
+        if (q < C::LOADS / 2) {
             const int r = 16 * I + (l >> 2), ch = (l & 3) ^ ((r >> 2) & 3);
             const int row = min(by * BM + r, p.m - 1);
             coff[q] = (uint32_t)(((size_t)row * p.k + ub * 32 + ch * 8) * 2);
@@ -172,8 +162,7 @@ __device__ __forceinline__ void gemm_big_tile(const GemmParams& p, int task, cha
     auto issue_one = [&](int ks, int buf, int q) {
         char* st = lds + buf * C::STAGE;
         const int I = w + C::NWAVES * q;
-        if (!C::EVEN && I >= C::NCOPY) return;
-        if (C::EVEN ? q < C::LOADS / 2 : I < C::A_COPIES)
+        if (q < C::LOADS / 2)
             lds_bdma16<AX>(abuf, coff[q], st + I * 1024, ks * 64);
         else
             lds_bdma16<false>(wbuf, coff[q], st + C::A_BYTES + (I - C::A_BYTES / 1024) * 1024, ks * 4096);
@@ -191,13 +180,8 @@ __device__ __forceinline__ void gemm_big_tile(const GemmParams& p, int task, cha
         return *(const float4*)(wcols + a * C::WN + 64 * j + 32 * h + 8 * q + 4 * hi);
     };
 
-    // This wave's copies a stage: LOADS, or LOADS - 1 (a wave-uniform branch between the waits).
-    const bool full_wave = C::EVEN || w < C::FULL;
-    if (nkt > 2) {
-        if (full_wave) wait_vmcnt<2 * C::LOADS>(); else wait_vmcnt<2 * C::LOADS - 2>();
-    } else {
-        if (full_wave) wait_vmcnt<C::LOADS>(); else wait_vmcnt<C::LOADS - 1>();
-    }
+    if (nkt > 2) wait_vmcnt<2 * C::LOADS>();
+    else wait_vmcnt<C::LOADS>();
     mark(1);  // (not in the loop: the clock read is a scalar-memory operation, and with one of
               // those outstanding the compiler waits for every LDS read at once)
     auto col_out = [&](int a) {
@@ -284,12 +268,8 @@ __device__ __forceinline__ void gemm_big_tile(const GemmParams& p, int task, cha
         }
         __builtin_amdgcn_sched_barrier(0);
         if (NEXT) {
-            if (NEXT_LAST)
-                wait_vmcnt<0>();
-            else if (full_wave)
-                wait_vmcnt<C::LOADS>();
-            else
-                wait_vmcnt<C::LOADS - 1>();
+            if (NEXT_LAST) wait_vmcnt<0>();
+            else wait_vmcnt<C::LOADS>();
             __builtin_amdgcn_s_barrier();
         }
 #pragma unroll
@@ -405,7 +385,7 @@ __device__ __forceinline__ void gemm_big_tile(const GemmParams& p, int task, cha
     // the table (256 bytes a row).
     const char* table = lds;
     if (ROPE) {
-        constexpr int COPIES = C::TM / 4 / C::NWAVES;
+        constexpr int COPIES = C::BM / 4 / C::NWAVES;
         const auto tbuf = buffer_rsrc(p.rope, (uint32_t)p.rope_rows * 256u);
         uint32_t toff[COPIES];
 #pragma unroll

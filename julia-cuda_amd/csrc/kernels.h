@@ -96,8 +96,10 @@ struct AttnParams {
 namespace jh {
 
 struct GemmConfig {
-    int bm;      // rows per tile: 16, 32, 48, 64 (latency kernel) or 128, 192, 256 (throughput kernel)
+    int bm;      // rows per tile: 16, 32, 48, 64 (latency kernel), 128 (throughput kernel) or 192, 256
+                 // (wide throughput kernel)
     int splits;  // K splits, 1-8
+    int height = 0;  // the wide kernel, unsplit: rows per tile (160, 192, 224, 256) in bm's place
 };
 
 // Device scratch the split-K GEMMs and split-KV attention share (never at the same time).
@@ -131,6 +133,10 @@ struct Gemm {
     float* logits = nullptr;
 };
 
+// The 256-column tiles of a checked GEMM, bm rows high (160, 192, 224 or 256; K splits 192 or 256).
+void gemm_wide_launch(const GemmParams& p, int epi, int bm, hipStream_t stream);
+int wide_height(int m, int n, int cus);
+
 // Throws std::runtime_error when g or cfg break what the kernels assume.
 void gemm_check(const Gemm& g, GemmConfig cfg, const Scratch& s);
 void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t stream);
@@ -138,6 +144,8 @@ void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t st
 // (the throughput tiles only where they take the epilogue: LayerNorm up to k = GEMM_BIG_LN_MAX_K).
 GemmConfig gemm_choose(int m, int n, int k, int cus, int epi = 0);
 constexpr int GEMM_BIG_LN_MAX_K = 1024;
+// gemm_choose's pick as it is run: a throughput tile's kernel and height.
+GemmConfig gemm_pick(int m, int n, int k, int cus, int epi = 0);
 // Compute units of the current device (queried once per device; 256 if the query fails).
 int device_cus();
 size_t gemm_ws_floats(int m, int n, GemmConfig cfg);

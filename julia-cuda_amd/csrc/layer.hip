@@ -28,6 +28,7 @@
 #include "attn_tile.h"
 #include "gemm_big.h"
 #include "gemm_tile.h"
+#include "gemm_wide.h"
 #include "layer.h"
 #include "rowops.h"
 
@@ -224,15 +225,17 @@ constexpr bool T48 = MODE == MODE_LAT48 && (EPI == EPI_K_ROPE || EPI == EPI_K_LN
 template <int EPI, bool AX, int MODE>
 __device__ __forceinline__ void gemm_phase(const GemmParams& g, int bm, char* lds, bool pre,
                                            uint32_t* s_last, uint64_t* sub) {
+    if (MODE == MODE_BIG256) {
+        gemm_wide_run<256, EPI, AX, true>(g, blockIdx.x, gridDim.x, lds, sub);
+        return;
+    }
     const int T = gemm_tasks(g);
     for (int t = blockIdx.x; t < T; t += gridDim.x) {
         const bool first = t == (int)blockIdx.x;
         const bool ready = pre && first;
         uint64_t* su = first ? sub : nullptr;
-        if (MODE == MODE_BIG256)
-            gemm_big_tile<256, 256, EPI, AX, true>(g, t, lds, su);
-        else if (MODE == MODE_BIG128 || bm == 128)
-            gemm_big_tile<128, 128, EPI, AX, true>(g, t, lds, su);
+        if (MODE == MODE_BIG128 || bm == 128)
+            gemm_big_tile<EPI, AX, true>(g, t, lds, su);
         else if (bm == 16)
             gemm_w_tile<16, EPI, AX>(g, t, lds, ready, s_last, su);
         else if (bm == 32)
@@ -436,14 +439,14 @@ int LayerKernel::lds_bytes(const LayerPlan& plan, int d, int inter, int m, int w
                       att_lds_bytes(attention_gkeys(m, window))});
     if (att_use_stream(m, 0) || att_use_stream(m, window)) b = std::max(b, ATT_STREAM_LDS);
     for (int g = 0; g < 4; g++)
-        b = plan.bm[g] >= 128 ? std::max(b, Big<128, 128>::LDS_BYTES)
+        b = plan.bm[g] >= 128 ? std::max(b, Big::LDS_BYTES)
                               : std::max({b, w_tile_bytes(ks[g], plan.splits[g]), red_bytes(plan.bm[g])});
     return (b + 15) / 16 * 16;
 }
 
 // The large-batch instances' LDS: the throughput tile or the streaming attention tile.
 static int big_lds_bytes(int bm) {
-    const int g = bm == 256 ? Big<256, 256>::LDS_BYTES : Big<128, 128>::LDS_BYTES;
+    const int g = bm == 256 ? Wide<256>::LDS_BYTES : Big::LDS_BYTES;
     return (std::max<int>(g, ATT_STREAM_LDS) + 15) / 16 * 16;
 }
 
@@ -522,7 +525,7 @@ static bool head_plan(const LayerPlan& plan, int m, int d, int ff, int cus, int 
     for (int g = 0; g < 5; g++) {
         if (mode != MODE_LAT) {
             const int t = mode == MODE_BIG256 ? 256 : 128;
-            if (cols[g] % t || ks[g] % 64 || (ln[g] && ks[g] > 128 * BIG_LN_SLOTS)) return false;
+            if (cols[g] % t || ks[g] % 64 || (ln[g] && ks[g] > GEMM_BIG_LN_MAX_K)) return false;
             bm[g] = t, splits[g] = 1;
         } else {
             lat_tile(m, cols[g], ks[g], cus, lds_max, bm[g], splits[g]);
@@ -546,7 +549,7 @@ LayerPlan LayerKernel::default_plan(int m, int d, int inter) const {
         // 256 x 256 where every GEMM's columns allow it (big_tiles below), else 128 x 128.
         const bool ln = g == 0 || g == 2;
         if (m > ATT_SLICE_ROWS && cols[g] % 128 == 0 && ks[g] % 64 == 0 &&
-            (!ln || ks[g] <= 128 * BIG_LN_SLOTS) && Big<128, 128>::LDS_BYTES <= lds_max_) {
+            (!ln || ks[g] <= GEMM_BIG_LN_MAX_K) && Big::LDS_BYTES <= lds_max_) {
             p.bm[g] = 128, p.splits[g] = 1;
             continue;
         }

@@ -4,7 +4,7 @@ instances within one dispatch summed, as rocprofv3 reports them).
 
     rocprofv3 --pmc MfmaUtil MfmaFlopsF16 SQ_BUSY_CYCLES -f csv -d OUT/mfma -o pmc -- \\
         python3 julia-cuda_amd/kernel_bench.py --step qkv --tokens 18752 --spec ...
-    python julia-cuda_amd/pmc_summary.py OUT/mfma --kernel "gemm_big<256, 20>" --kernel gemm_lat1
+    python julia-cuda_amd/pmc_summary.py OUT/mfma --kernel "gemm_wide<224, 20" --kernel gemm_lat1
 
 Prints one JSON object: {kernel: {"dispatches": n, counter: median, ...}}. With --duration-us
 KERNEL=US (the kernel's average duration from a --kernel-trace --stats run), MfmaFlopsF16 is

@@ -207,6 +207,24 @@ def test_big_tiles_every_epilogue(torch_cuda, scratch, kind, n, k, bm):
     check_gemm(P, out, st, f"{kind} M=2100 n={n} k={k} bm={bm}")
 
 
+# The wide tiles. bm 0: at these sizes the pick on 256 CUs, 160, 192, 224 and 256 rows high, a
+# row past a whole tile or so, one round; the last two with two tasks a block, whose stage copies run
+# on over the tasks (13 stages of 64: the second task starts in the other stage space). bm given:
+# tasks of one, two and three stages, two a block.
+WIDE = [("lngeglu", 4321, 2304, 768, 0), ("lnrope", 5001, 2304, 768, 0), ("resstats", 5185, 2304, 768, 0),
+        ("lnbias", 6001, 2304, 768, 0), ("lngeglu", 7001, 2304, 768, 0), ("lnrope", 9001, 2304, 832, 0),
+        ("resstats", 9001, 2304, 832, 0), ("lnrope", 30011, 768, 64, 256), ("resstats", 30011, 768, 64, 192),
+        ("lnrope", 30011, 768, 128, 192), ("lngeglu", 30011, 768, 192, 256), ("biasresstats", 1, 256, 64, 256)]
+
+
+@pytest.mark.parametrize("kind,m,n,k,bm", WIDE, ids=["-".join(map(str, w)) for w in WIDE])
+def test_wide_tile_heights_and_streams(torch_cuda, scratch, kind, m, n, k, bm):
+    say(f"wide tiles {kind} M={m} N={n} K={k} bm={bm}")
+    P = gemm_problem(kind, m, n, k, seed=81 + m + k)
+    out, st = run_gemm(torch_cuda, P, bm, 1, scratch)
+    check_gemm(P, out, st, f"{kind} m={m} n={n} k={k} bm={bm}")
+
+
 @pytest.mark.parametrize("kind,n,k", [("lnrope", 2304, 768), ("resstats", 768, 1152),
                                       ("lngeglu", 2304, 768), ("lnbiasgelu", 768, 768)])
 def test_chooser_at_row_edges(torch_cuda, scratch, kind, n, k):
