@@ -467,13 +467,13 @@ __device__ __forceinline__ void attention_slice_tile(const AttnParams& p, int ta
 // rows' sequences and the window) goes through two LDS stages of 64 keys, K and V row-major and
 // swizzled as in the slice tile, filled by direct global -> LDS loads one block ahead of the
 // MFMAs; a 64-key block is two of the slice tile's 32-key steps. Each key is read once per 64
-// queries, and with four blocks a CU (32 KB of LDS and 108 registers a lane each) the waves
+// queries, and with five blocks a CU (32 KB of LDS and 96 registers a lane each) the waves
 // hide each other's step latencies.
 //
 // KS = 2 or 4 (one long sequence, a grid of about a block a CU): the block has KS groups of NW
 // waves, each running the online softmax of the same NW x 16 queries over every KS-th key
 // block (group g takes blocks g, g + KS, ...) through its own stage ring, in lockstep (one
-// block barrier a step for all); groups 1 .. KS - 1 then pass their running max, sum and
+// block barrier a step for all); groups 1 .. KS - 1 then pass their max, sum and
 // output through LDS and group 0 merges them (in group order: deterministic). Two or four
 // waves a SIMD instead of one hide each other's step latencies where the grid leaves the CUs
 // a block each, and the chain of steps is KS times shorter. NW = 1, KS = 4 (short inputs: a
@@ -482,61 +482,72 @@ __device__ __forceinline__ void attention_slice_tile(const AttnParams& p, int ta
 constexpr int ATT_STREAM_STAGES = 2;
 constexpr int ATT_STREAM_LDS = ATT_STREAM_STAGES * 16384;
 
-// One 64-key block of the streaming tile for a wave's 16 queries (lane l: query l % 16): S^T for
-// keys kb + 16 t + 4 g + e (t < 4) from the block's K fragments, one max and one rescale, P . V in
-// two K-32 halves. full: every score is valid; else key kb + 16 t + 4 g + e is valid iff
-// (uint32_t)(base + 16 t + e) < kspan, base = kb + 4 g - (the lane's first valid key).
-__device__ __forceinline__ void att_stream_block(const half8 (&kf)[4][2], const half4 (&vlo)[2][4],
-                                                 const half4 (&vhi)[2][4], const half8 (&qf)[2],
-                                                 bool full, int base, uint32_t kspan, float& mx,
-                                                 float& lsum, floatx4 (&oacc)[4]) {
-    const float scale = 1.4426950408889634f / 8.0f;  // log2(e) / sqrt(64)
-    floatx4 sc[4];
+constexpr float ATT_SCALE = 1.4426950408889634f / 8.0f;  // log2(e) / sqrt(64)
+
+// The online softmax's state of a lane's query (the same in the four lanes that share it, but for
+// the sum, which covers the lane's own keys): the weights are exp2(score scale - max scale), so the
+// largest is 1 and exact in f16.
+//
+// Where no score of the wave's block exceeds its query's maximum, a block takes no maximum across
+// lanes, no exponential of its change and no rescale, which on random scores is about half of a long
+// sequence's blocks. A maximum that may lag by some powers of two would spare nearly all (2029 rows
+// 22.0 us), but leaves the largest weight rounded: up to 30% more error on peaked scores.
+//
+// What bounds the tile is the VALU: a wave's 64-key block took ~640 clocks of it (125 operations, 17
+// of them exponentials of 16 clocks each; its MFMAs 256 clocks) and takes ~510 where it skips the
+// rescale. With V's fragments read behind S^T's MFMAs and without the copies of the scores where the
+// masked and the full path join: 2029 rows 27.0 -> 25.4 us, 4096 rows 79.7 -> 75.2, config 5's batch
+// 53.7 -> 50.3 a global layer.
+struct AttState {
+    float top = -INFINITY;   // the maximum, unscaled; -inf: no valid key yet
+    float mx = -INFINITY;    // top x ATT_SCALE
+    float neg = 0.0f;        // -mx, 0 while there is none (exp2(-inf) = 0 then)
+    float sum = 0.0f;
+    floatx4 o[4];
+};
+
+// One 64-key block of the streaming tile for a wave's 16 queries (lane l: query l % 16): the
+// softmax and P . V (two K-32 halves) of its scores sc (keys kb + 16 t + 4 g + e, t < 4). full: every
+// score is valid; else key kb + 16 t + 4 g + e is valid iff (uint32_t)(base + 16 t + e) < kspan,
+// base = kb + 4 g - (the lane's first valid key).
+__device__ __forceinline__ void att_stream_block(floatx4 (&sc)[4], const half4 (&vlo)[2][4],
+                                                 const half4 (&vhi)[2][4], bool full, int base,
+                                                 uint32_t kspan, AttState& a) {
+    if (!full) {
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
-        sc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < 4; t++)
 #pragma unroll
-        for (int k2 = 0; k2 < 2; k2++) sc[t] = mfma16(kf[t][k2], qf[k2], sc[t]);
+            for (int e = 0; e < 4; e++)
+                sc[t][e] = (uint32_t)(base + 16 * t + e) < kspan ? sc[t][e] : -INFINITY;
     }
+    // (The four scores as one register group where the paths join: the compiler otherwise copies
+    // each of the 16 into a register of its own in the full path.)
+#pragma unroll
+    for (int t = 0; t < 4; t++) asm volatile("" : "+v"(sc[t]));
     float bm = -INFINITY;
-    if (full) {
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+    for (int t = 0; t < 4; t++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                bm = fmaxf(bm, sc[t][e]);
-            }
-    } else {
+        for (int e = 0; e < 4; e++) bm = fmaxf(bm, sc[t][e]);
+    if (__builtin_amdgcn_ballot_w64(bm > a.top) != 0) {  // (wave-uniform)
+        a.top = fmaxf(a.top, max_xor32(max_xor16(bm)));
+        const float m = a.top * ATT_SCALE, b0 = m == -INFINITY ? 0.0f : m;
+        const float alpha = fast_exp2(a.mx - b0);
+        a.mx = m;
+        a.neg = -b0;
+        a.sum *= alpha;
 #pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const bool ok = (uint32_t)(base + 16 * t + e) < kspan;
-                sc[t][e] = ok ? sc[t][e] : -INFINITY;
-                bm = fmaxf(bm, sc[t][e]);
-            }
+        for (int dt = 0; dt < 4; dt++) a.o[dt] = a.o[dt] * alpha;
     }
-    bm = max_xor32(max_xor16(bm)) * scale;  // the scores stay unscaled until the exponent
-    const float mnew = fmaxf(mx, bm);
-    const float b0 = mnew == -INFINITY ? 0.0f : mnew;  // no valid key yet: exp2(-inf) = 0
-    const float alpha = fast_exp2(mx - b0);
-    // The output needs rescaling only where a lane's max rose (alpha < 1): skipped when no lane
-    // of the wave has (a wave-uniform test).
-    const bool rescale = __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0;
-    mx = mnew;
     float rs = 0.0f;
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            sc[t][e] = fast_exp2(fmaf(sc[t][e], scale, -b0));
+            sc[t][e] = fast_exp2(fmaf(sc[t][e], ATT_SCALE, a.neg));
             rs += sc[t][e];
         }
-    lsum = lsum * alpha + rs;
-    if (rescale) {
-#pragma unroll
-        for (int dt = 0; dt < 4; dt++) oacc[dt] = oacc[dt] * alpha;
-    }
+    a.sum += rs;
 #pragma unroll
     for (int hf = 0; hf < 2; hf++) {
         half8 pf;
@@ -549,7 +560,7 @@ __device__ __forceinline__ void att_stream_block(const half8 (&kf)[4][2], const 
         for (int dt = 0; dt < 4; dt++) {
             const half4 lo = vlo[hf][dt], hi = vhi[hf][dt];
             const half8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            oacc[dt] = mfma16(vf, pf, oacc[dt]);
+            a.o[dt] = mfma16(vf, pf, a.o[dt]);
         }
     }
 }
@@ -561,8 +572,8 @@ template <bool XS = false, int NW = 4, int KS = 1>
 __device__ __forceinline__ void attention_stream_tile(const AttnParams& p, int task, char* lds) {
     static_assert(KS == 1 || KS == 2 || KS == 4, "key groups");
     constexpr int NS = ATT_STREAM_STAGES, QB = 16 * NW;
-    constexpr int LOADS = 16 / NW;  // 1 KB copies a wave per stage
-    static_assert(NW == 1 || NW == 2 || NW == 4 || NW == 8, "waves");
+    constexpr int LOADS = (16 + NW - 1) / NW;  // 1 KB copies a wave per stage (six waves: three or two)
+    static_assert(NW == 1 || NW == 2 || NW == 4 || NW == 6 || NW == 8, "waves");
     const int n = p.n, d = p.d, ld = 3 * d, heads = d >> 6;
     const int tiles = (n + QB - 1) / QB;
     const int L = xcd_task(task, tiles * heads);
@@ -595,10 +606,13 @@ __device__ __forceinline__ void attention_stream_tile(const AttnParams& p, int t
     // (c % 8) ^ (row % 8). The copies go through a buffer descriptor over the block's rows: the
     // lane's offsets within a block are fixed (computed once), and rows past n read as zeros
     // (their keys are masked).
+    auto is_k = [&](int qq) {  // copy w + NW qq of the 16 is K's: the first half of a wave's copies
+        return 16 % NW == 0 ? qq < LOADS / 2 : w + NW * qq < 8;
+    };
     uint32_t doff[LOADS];
 #pragma unroll
     for (int qq = 0; qq < LOADS; qq++) {
-        const bool kk = qq < LOADS / 2;  // the first half of a wave's copies are K's
+        const bool kk = is_k(qq);
         const int I = (w + NW * qq) & 7;
         const int c = I * 64 + l, row = c >> 3, ch = (c & 7) ^ (row & 7);
         doff[qq] = (uint32_t)((row * ld + (kk ? d : 2 * d) + h * 64 + ch * 8) * 2);
@@ -610,7 +624,8 @@ __device__ __forceinline__ void attention_stream_tile(const AttnParams& p, int t
                                     (uint32_t)(min(n - kb, 64) * ld * 2));
 #pragma unroll
         for (int qq = 0; qq < LOADS; qq++) {
-            const bool kk = qq < LOADS / 2;
+            if (16 % NW != 0 && w + NW * qq >= 16) break;  // (wave-uniform)
+            const bool kk = is_k(qq);
             const int I = (w + NW * qq) & 7;
             lds_bdma16<false>(rs, doff[qq], dst + (kk ? 0 : 8192) + I * 1024);
         }
@@ -641,10 +656,9 @@ __device__ __forceinline__ void attention_stream_tile(const AttnParams& p, int t
         qf[1] = load16h<false>(qp + 32);
     }
 
-    float mx = -INFINITY, lsum = 0.0f;
-    floatx4 oacc[4];
+    AttState a;
 #pragma unroll
-    for (int t = 0; t < 4; t++) oacc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int t = 0; t < 4; t++) a.o[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
     // The lane's LDS offsets within a stage, loop-invariant: with the stage a constant in each
     // unrolled step below, every read is a base register plus an immediate. (Rows 16 t, and
@@ -658,10 +672,11 @@ __device__ __forceinline__ void attention_stream_tile(const AttnParams& p, int t
 
     // The group's step b: its block kg + KS b (if there is one), in stage ST = b % NS (a
     // constant). Both groups take every step: the barrier is the block's. A step waits for its
-    // block's copies (the only ones in flight), issues every LDS read of the block, then copies
-    // the next block into the other stage and computes while that copy flies: the compiler
-    // makes any LDS read wait for every direct-to-LDS copy in flight (it cannot tell the stages
-    // apart), so a copy issued before a read would be waited for there.
+    // block's copies (the only ones in flight), reads K's fragments, issues S^T's MFMAs and reads
+    // V's fragments behind them (used after the softmax), then copies the next block into the
+    // other stage and computes while that copy flies: the compiler makes any LDS read wait for
+    // every direct-to-LDS copy in flight (it cannot tell the stages apart), so a copy issued
+    // before a read would be waited for there.
     const int nsteps = (nblk + KS - 1) / KS;
     auto has = [&](int b) { return kg + KS * b < nblk; };
     auto step = [&](int b, auto st_) {
@@ -673,15 +688,23 @@ __device__ __forceinline__ void attention_stream_tile(const AttnParams& p, int t
         const int kb = k0 + 64 * (kg + KS * b);
         const bool act = has(b) && !(kb + 64 <= wlo || kb >= whi);
         const char* st = ring + ST * 16384;
-        // The 64 keys in one step: S^T for keys kb + 16 t + 4 g + e (t < 4), one max and one
-        // rescale; P . V in two K-32 halves.
-        half8 kf[4][2];
+        // S^T for keys kb + 16 t + 4 g + e (t < 4) of the lane's query.
+        floatx4 sc[4];
         half4 vlo[2][4], vhi[2][4];
         if (act) {
+            half8 kf[4][2];
 #pragma unroll
             for (int t = 0; t < 4; t++)
 #pragma unroll
                 for (int k2 = 0; k2 < 2; k2++) kf[t][k2] = *(const half8*)(st + koff[k2] + 2048 * t);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                sc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int k2 = 0; k2 < 2; k2++) sc[t] = mfma16(kf[t][k2], qf[k2], sc[t]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int hf = 0; hf < 2; hf++)
 #pragma unroll
@@ -696,7 +719,7 @@ __device__ __forceinline__ void attention_stream_tile(const AttnParams& p, int t
         if (!act) return;
         const bool full = one_seq && kb >= ulo && kb + 64 <= uhi &&
                           (p.window == 0 || (wql - kb <= p.window && kb + 63 - wq0 <= p.window));
-        att_stream_block(kf, vlo, vhi, qf, full, kb + 4 * g - klo, kspan, mx, lsum, oacc);
+        att_stream_block(sc, vlo, vhi, full, kb + 4 * g - klo, kspan, a);
     };
 
     static_assert(NS == 2, "the loop below is unrolled by the stages");
@@ -707,47 +730,47 @@ __device__ __forceinline__ void attention_stream_tile(const AttnParams& p, int t
     }
 
     if (KS > 1) {
-        // Groups 1 .. KS - 1: running max, sum and unnormalised output into the first rings
+        // Groups 1 .. KS - 1: max, sum and unnormalised output into the first rings
         // (every wave is done with the stages: the barrier); group 0 merges them with its own,
         // in group order (deterministic).
         auto slot = [&](int k) { return (float*)lds + (size_t)((k - 1) * NW + w) * 18 * 64; };
         __syncthreads();
         if (kg > 0) {
             float* mg = slot(kg);
-            mg[16 * 64 + l] = mx;
-            mg[17 * 64 + l] = lsum;
+            mg[16 * 64 + l] = a.mx;
+            mg[17 * 64 + l] = a.sum;
 #pragma unroll
             for (int dt = 0; dt < 4; dt++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) mg[(4 * dt + e) * 64 + l] = oacc[dt][e];
+                for (int e = 0; e < 4; e++) mg[(4 * dt + e) * 64 + l] = a.o[dt][e];
         }
         __syncthreads();
         if (kg > 0) return;  // (their threads take no further barrier)
         float mk[KS];
-        mk[0] = mx;
+        mk[0] = a.mx;
 #pragma unroll
         for (int k = 1; k < KS; k++) mk[k] = slot(k)[16 * 64 + l];
-        float m = mx;
+        float m = a.mx;
 #pragma unroll
         for (int k = 1; k < KS; k++) m = fmaxf(m, mk[k]);
         const float base = m == -INFINITY ? 0.0f : m;
-        const float a0 = fast_exp2(mx - base);
-        lsum = lsum * a0;
+        const float a0 = fast_exp2(a.mx - base);
+        a.sum = a.sum * a0;
 #pragma unroll
-        for (int dt = 0; dt < 4; dt++) oacc[dt] = oacc[dt] * a0;
+        for (int dt = 0; dt < 4; dt++) a.o[dt] = a.o[dt] * a0;
 #pragma unroll
         for (int k = 1; k < KS; k++) {
             const float* mg = slot(k);
             const float ak = fast_exp2(mk[k] - base);
-            lsum += mg[17 * 64 + l] * ak;
+            a.sum += mg[17 * 64 + l] * ak;
 #pragma unroll
             for (int dt = 0; dt < 4; dt++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) oacc[dt][e] += mg[(4 * dt + e) * 64 + l] * ak;
+                for (int e = 0; e < 4; e++) a.o[dt][e] += mg[(4 * dt + e) * 64 + l] * ak;
         }
     }
 
-    const float tot = sum_xor32(sum_xor16(lsum));
+    const float tot = sum_xor32(sum_xor16(a.sum));
     const float inv = tot > 0.0f ? 1.0f / tot : 0.0f;
     if (qi < n) {
         f16* op = (f16*)p.o + (size_t)qi * d + h * 64 + 4 * g;
@@ -755,7 +778,7 @@ __device__ __forceinline__ void attention_stream_tile(const AttnParams& p, int t
         for (int dt = 0; dt < 4; dt++) {
             half4 ov;
 #pragma unroll
-            for (int e = 0; e < 4; e++) ov[e] = (f16)(oacc[dt][e] * inv);
+            for (int e = 0; e < 4; e++) ov[e] = (f16)(a.o[dt][e] * inv);
             store8<XS>(op + 16 * dt, ov);
         }
     }

@@ -330,6 +330,30 @@ def test_attention_d384_and_tail(torch_cuda, scratch):
         compare(f32(f16_bits(o)), ref, ATTN_REL, what=f"attention d=384 n={n} w={window}")
 
 
+@pytest.mark.parametrize("n", [300, 600, 1000, 1344, 1345, 2016, 2017, 2731])
+@pytest.mark.parametrize("window", [0, 64])
+@pytest.mark.parametrize("rise", [-90.0, 6.0, 90.0])
+def test_attention_moving_maximum(torch_cuda, scratch, n, window, rise):
+    """The streaming tile's running maximum: scores that rise (or fall) along the keys by `rise` in the
+    exp2 domain, so that only a query's first block moves it, some blocks or nearly every one, on each
+    instance of the tile (four single-wave key groups, 2 x 4, 4 x 4, 6 x 2 at its smallest and
+    largest, 4 x 2, 4 x 1), against the f64 attention."""
+    torch = torch_cuda
+    rng = np.random.default_rng(40 + n)
+    x = rng.standard_normal((n, 3, 12, 64)).astype(np.float32)
+    # q . k / 8 * log2(e) rises by `rise` over the n keys through dimension 0 (q there: 8)
+    x[:, 0, :, 0] = 8.0
+    x[:, 1, :, 0] = (np.arange(n) / n * rise / 1.4426950408889634)[:, None]
+    qkv16 = O.to_f16_bits(x.reshape(n, 3 * 768))
+    ref = O.attention(f32(qkv16), window)
+    q = to_dev(torch, qkv16)
+    o = torch.full((n, 768), float("nan"), dtype=torch.float16, device="cuda")
+    jh.attention(q.data_ptr(), o.data_ptr(), n, 768, window, 1, scratch,
+                 stream=torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    compare(f32(f16_bits(o)), ref, ATTN_REL, what=f"attention n={n} w={window} rise={rise}")
+
+
 @pytest.mark.parametrize("window", [0, 64])
 def test_attention_at_the_routing_edges(torch_cuda, scratch, window):
     """One sequence at d=768 on both sides of every size where attention_launch changes tile
