@@ -173,6 +173,10 @@ void embed_launch(const uint32_t* ids, int n, const jh_half* table, int vocab, i
 void norm_add_launch(const jh_half* x, int n, int d, const float* gamma, const float* add,
                      float eps, jh_half* out, float* stats, hipStream_t stream,
                      const int32_t* row_type = nullptr);
+// Per row of a concatenated batch its position in its request, its request's rows [first, one past
+// last) and question type; table: each request's first row, rows (1 at least) and question type.
+void batch_rows_launch(const uint32_t* table, int requests, int32_t* pos, int32_t* seg, int32_t* type,
+                       hipStream_t stream);
 // Rows markers[i] (i < k) of a, and of b and the row statistics when given, into row i of
 // a_out (b_out, stats_out).
 void gather_rows_launch(const jh_half* a, const jh_half* b, const float* stats, int n, int d,

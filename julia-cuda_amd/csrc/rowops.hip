@@ -58,6 +58,19 @@ __global__ __launch_bounds__(256) void score_kernel(const f16* y, int n, int d, 
     score_row<NC>(y, n, d, w, b, markers, i, logits, threadIdx.x & 63);
 }
 
+// A block a request of a concatenated batch: its rows' positions, sequence bounds and question
+// type, from the table's (first row, rows, question type).
+__global__ __launch_bounds__(256) void batch_rows_kernel(const uint32_t* table, int32_t* pos, int2* seg,
+                                                         int32_t* type) {
+    const uint32_t* t = table + 3 * (size_t)blockIdx.x;
+    const int r0 = (int)t[0], rows = (int)t[1], q = (int)t[2];
+    for (int i = threadIdx.x; i < rows; i += 256) {
+        pos[r0 + i] = i;
+        seg[r0 + i] = make_int2(r0, r0 + rows);
+        type[r0 + i] = q;
+    }
+}
+
 // dst = src, 16 bytes per thread per step, grid-stride: the plain copy kernel the byte counters
 // (rocprofv3 FETCH_SIZE / WRITE_SIZE) are calibrated against, and the achievable-bandwidth
 // probe for the bandwidth-bound kernels.
@@ -140,6 +153,13 @@ void gather_rows_launch(const jh_half* a, const jh_half* b, const float* stats, 
                        (const uint4*)b, (const float2*)stats, n, d, markers, k, (uint4*)a_out,
                        (uint4*)b_out, (float2*)stats_out);
     check_launch("gather");
+}
+
+void batch_rows_launch(const uint32_t* table, int requests, int32_t* pos, int32_t* seg, int32_t* type,
+                       hipStream_t st) {
+    if (requests <= 0) return;
+    hipLaunchKernelGGL(batch_rows_kernel, dim3(requests), dim3(256), 0, st, table, pos, (int2*)seg, type);
+    check_launch("batch rows");
 }
 
 void score_launch(const jh_half* y, int n, int d, const jh_half* w, float b,

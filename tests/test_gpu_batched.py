@@ -131,6 +131,23 @@ def test_full_pass_of_max_length_requests(engine):
     path_diff(got, alone, "full passes")
 
 
+@pytest.mark.parametrize("lens", [(1, 255, 256, 257, 1, 512, 2), (1,) * ROWS])
+def test_batch_rows_at_the_edges(engine, lens):
+    """The per-row arrays of a pass, written from the table of its requests by a block of 256 threads
+    each: requests of a row, of a block's rows and one either side, and as many requests as the engine
+    has rows (the fullest table), with markers on first and last rows and the types in turn."""
+    e, _ = engine
+    rng = np.random.default_rng(len(lens))
+    reqs = []
+    for i, n in enumerate(lens):
+        ids = rng.integers(0, SMALL["vocab"], n).astype(np.uint32)
+        reqs.append((ids, np.array([0, n - 1], np.uint32), i % 3))
+    got, ms = e.run(reqs, batched=True)
+    assert np.all(ms == ms[0])
+    alone, _ = e.run(reqs[:20])
+    path_diff(got[:20], alone, f"{len(lens)} requests")
+
+
 def test_many_markers(engine):
     """A request may name a marker any number of times (src/engine.rs:78-81 only bounds the
     positions): more markers than max_length, through the graph path, the direct path and the
