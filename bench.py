@@ -208,8 +208,13 @@ def path_ms(t):
 def gemm_instance(m, n, k, bm, epi, cus):
     """The kernel instance the engine launches for an m x n x k GEMM with tile height bm (one
     K split)."""
+    ks, ceil = k / 768, lambda a, b: -(-a // b)
+    lines = max(2, ceil(k // 64, 4))  # the grouped latency kernel's instance and its highest tile
+    top = {2: 128, 3: 96, 4: 64, 5: 64, 6: 48}.get(lines, 0) if k >= 256 else 0
+    for h in (16, 32, 48, 64, 80, 96, 128):
+        if h <= top and n // 64 * ceil(m, h) <= cus:
+            return f"gemm_group<{h}, {jh.EPI[epi]}, {lines}>"
     if bm >= 128:  # the throughput kernel the launch takes (gemm_pick in csrc/gemm.hip)
-        ks, ceil = k / 768, lambda a, b: -(-a // b)
         l128 = ceil(n // 128 * ceil(m, 128), cus)
         c128 = 2 + 8.5 * ks if l128 == 1 else 2.5 + 7.6 * ks * l128
         rounds = lambda h: ceil(n // 256 * ceil(m, h), cus)
@@ -218,9 +223,7 @@ def gemm_instance(m, n, k, bm, epi, cus):
             return f"gemm_wide<{h}, {jh.EPI[epi]}, false>"
         return f"gemm_big<{jh.EPI[epi]}, false>"
     if (n // 64) * -(-m // bm) <= cus and k >= 256:  # the eight-wave instance: a block a CU at most
-        most = (k // 32 + 7) // 8  # K steps of the busiest wave: its K path
-        path = 3 if most <= 3 else 5 if most <= 5 else 6 if most <= 6 and bm <= 32 else 1
-        return f"gemm_lat1<{bm}, {jh.EPI[epi]}, {path}>"
+        return f"gemm_lat1<{bm}, {jh.EPI[epi]}>"
     return f"gemm_lat<{bm}, {jh.EPI[epi]}>"
 
 

@@ -3,15 +3,14 @@
 // kernels/src/main.rs:886-1041) walks K through shared tiles with 4-8 warps each owning a
 // piece of the output; here two kernels cover the two regimes of a 256-CU GPU:
 //
-//  - gemm_lat / gemm_lat1 (BM = 16/32/48/64 rows x 64 columns): the small-M, latency-bound
-//    regime of one request (M = 72-1024). The block's waves split K between them and reduce
-//    their partial tiles through LDS, so a tile's serial K loop is short and there are more
-//    tiles to spread over 256 CUs. gemm_lat1, for grids of at most a block a CU (every latency
-//    GEMM of a 293-token request), runs eight waves, copies each wave's range of a into LDS as
-//    whole 128-byte lines and fixes the waves' K path per kernel instance (gemm_tile.h);
-//    gemm_lat runs four waves streaming a and w fragments from L2 into registers, two blocks a
-//    CU. Grid split-K on top is deterministic: the last block of a tile to arrive sums every
-//    split's partial in split order.
+//  - gemm_group (16 to 128 rows x 64 columns, gemm_group.h): the latency-bound regime, grids of at
+//    most a block a CU (every GEMM of a request of up to 672 tokens): eight waves in four K groups,
+//    a's rows whole in LDS, w straight into registers, the partial tiles summed through LDS.
+//  - gemm_lat (BM = 16/32/48/64 rows x 64 columns): more tiles than CUs, or a K split. The block's
+//    four waves split K between them, streaming a and w fragments from L2 into registers, two
+//    blocks a CU. Grid split-K on top is deterministic: the last block of a tile to arrive sums
+//    every split's partial in split order. gemm_lat1, its eight-wave form on a CU of its own, is
+//    left for the K that gemm_group does not hold (past 1536).
 //  - gemm_big (128 x 128 tiles): the middle sizes and widths that 256 does not divide: a and w
 //    tiles copied into four LDS stages by direct buffer -> LDS loads (gemm_big.h), four waves each
 //    owning a 64 x 64 output block on 32 x 32 x 16 MFMA, the epilogue's column-wise part applied on
@@ -45,17 +44,15 @@ __global__ __launch_bounds__(256, 2) void gemm_lat(GemmParams p) {
     gemm_lat_tile<BM, EPI>(p, blockIdx.x, red, &s_last);
 }
 
-// gemm_lat for grids of at most one block a CU (one request's GEMMs up to ~300 tokens): eight
-// waves split the tile's K steps, each issuing all of its three to five steps' loads at once. A
-// CU takes in its operands from L2 faster with eight waves loading than with four (measured on
-// MI355X: ~86-94 against ~55-79 GB/s), for twice the partial tiles to sum through LDS. KP: the
-// waves' K path (LAT_KONE3 / 5 / 6, LAT_KLOOP), chosen by the host from K and BM. Dynamic LDS:
-// lat_lds_floats<BM, 8>() floats.
-template <int BM, int EPI, int KP>
+// gemm_lat for grids of at most one block a CU, where gemm_group does not take K: eight waves split
+// the tile's K steps. A CU takes in its operands from L2 faster with eight waves loading than with
+// four (measured on MI355X: ~86-94 against ~55-79 GB/s), for twice the partial tiles to sum through
+// LDS. Dynamic LDS: lat_lds_floats<BM, 8>() floats.
+template <int BM, int EPI>
 __global__ __launch_bounds__(512, 1) void gemm_lat1(GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) float red_dyn[];
     __shared__ uint32_t s_last;
-    gemm_lat_tile<BM, EPI, false, false, 8, KP>(p, blockIdx.x, red_dyn, &s_last);
+    gemm_lat_tile<BM, EPI, false, 8>(p, blockIdx.x, red_dyn, &s_last);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -199,40 +196,22 @@ static void launch_big(const GemmParams& p, hipStream_t st) {
     hipLaunchKernelGGL((gemm_big<EPI, SPLIT>), dim3(grid), dim3(Big::THREADS), (Big::LDS_BYTES), st, p);
 }
 
-template <int BM, int EPI, int KP>
+template <int BM, int EPI>
 static void launch_lat1(const GemmParams& p, int blocks, hipStream_t st) {
     constexpr int LDS = lat_lds_floats<BM, 8>() * 4;
     static const bool lds_ok =  // once per instantiation, before its first launch
-        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_lat1<BM, EPI, KP>),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_lat1<BM, EPI>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS) == hipSuccess;
     if (!lds_ok) throw std::runtime_error("gemm: the one-block latency kernel cannot have its LDS");
-    hipLaunchKernelGGL((gemm_lat1<BM, EPI, KP>), dim3(blocks), dim3(512), LDS, st, p);
-}
-
-// The eight-wave kernel's K path for K and the tile height: wave w of 8 takes K steps
-// [w U / 8, (w + 1) U / 8) of U = K / 32, at most ceil(U / 8); six in one chunk for tiles of up
-// to 32 rows (K = 1536: the head's linear2, 6.8 us on the chunked loop).
-static int gemm_lat1_path(int k, int bm) {
-    const int most = (k / 32 + 7) / 8;
-    return most <= 3 ? LAT_KONE3 : most <= 5 ? LAT_KONE5 : most <= 6 && bm <= 32 ? LAT_KONE6 : LAT_KLOOP;
+    hipLaunchKernelGGL((gemm_lat1<BM, EPI>), dim3(blocks), dim3(512), LDS, st, p);
 }
 
 template <int BM, int EPI>
 static void launch_lat(const GemmParams& p, hipStream_t st) {
     const int blocks = p.tiles_n * p.tiles_m * p.splits;
     // (Eight waves with a K step each: K >= 256.)
-    if (p.splits == 1 && blocks <= device_cus() && p.k >= 256) {
-        switch (gemm_lat1_path(p.k, BM)) {
-            case LAT_KONE3: launch_lat1<BM, EPI, LAT_KONE3>(p, blocks, st); break;
-            case LAT_KONE5: launch_lat1<BM, EPI, LAT_KONE5>(p, blocks, st); break;
-            case LAT_KONE6:
-                if constexpr (BM <= 32) launch_lat1<BM, EPI, LAT_KONE6>(p, blocks, st);
-                break;
-            default: launch_lat1<BM, EPI, LAT_KLOOP>(p, blocks, st); break;
-        }
-    } else {
-        hipLaunchKernelGGL((gemm_lat<BM, EPI>), dim3(blocks), dim3(256), 0, st, p);
-    }
+    if (p.splits == 1 && blocks <= device_cus() && p.k >= 256) launch_lat1<BM, EPI>(p, blocks, st);
+    else hipLaunchKernelGGL((gemm_lat<BM, EPI>), dim3(blocks), dim3(256), 0, st, p);
 }
 
 // The epilogues only the latency tiles take (the score, gathered rows).
@@ -269,7 +248,10 @@ void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t st
     p.tiles_n = g.n / (cfg.bm >= 128 ? big_bn(cfg.bm) : 64);
     const int bm = cfg.height ? cfg.height : cfg.bm;
     p.tiles_m = (g.m + bm - 1) / bm;
-    switch (g.epi) {
+    const bool group = cfg.bm < 128 && cfg.splits == 1 && gemm_group_takes(bm, g.k) &&
+                       (cfg.height || p.tiles_n * p.tiles_m <= device_cus());
+    if (group) gemm_group_launch(p, g.epi, bm, st);
+    else switch (g.epi) {
         case EPI_K_ROPE: launch_epi<EPI_K_ROPE>(p, bm, st); break;
         case EPI_K_LNROPE: launch_epi<EPI_K_LNROPE>(p, bm, st); break;
         case EPI_K_LNGEGLU: launch_epi<EPI_K_LNGEGLU>(p, bm, st); break;
@@ -424,10 +406,13 @@ GemmConfig gemm_choose(int m, int n, int k, int cus, int epi) {
 // So 128 x 128 for qkv and wi up to ~3000 rows and for wo up to 8192 (17.5 us there against 18.5
 // for the wide tiles; wo_mlp level, 23.5), the wide tiles for qkv and wi from 4096 (18.5 us
 // against 25) and for everything at 18752.
+// And before these, wherever a grid of at most a block a CU covers the GEMM, the grouped latency
+// kernel at its smallest such height (gemm_group.hip has the figures).
 GemmConfig gemm_pick(int m, int n, int k, int cus, int epi) {
+    if (cus <= 0) cus = 256;
+    if (const int h = gemm_group_height(m, n, k, cus)) return GemmConfig{std::min(h, 64), 1, h};
     GemmConfig best = gemm_choose(m, n, k, cus, epi);
     if (best.bm < 128) return best;
-    if (cus <= 0) cus = 256;
     const double ks = (double)k / 768.0;
     const long l128 = ((long)(n / 128) * ((m + 127) / 128) + cus - 1) / cus;
     best = GemmConfig{128, 1};

@@ -1,0 +1,204 @@
+// One output tile of the grouped latency GEMM (BM rows x 64 columns), for grids of at most a block a
+// CU: eight waves in four K groups of two column halves.
+//
+// Bound by a launch and a first round trip (~2.5 us), then by how fast a CU takes in its operands: a
+// 48-row tile at K = 768 asks for 1344 lines of 128 bytes, about 2 ns each.
+//
+// a's rows of the tile go into LDS once, whole: K is cut on its 128-byte lines, group g taking lines
+// [g N / 4, (g + 1) N / 4) of the N = K / 64, copied by its two waves (half the rows each) as 8 rows x
+// one line a copy, ahead of any other load of the tile. Each wave's fragments of w (its K range's 32
+// columns) follow, straight into registers, all in flight at once. A CU takes in its operands in the
+// order they were asked for, so w's arrival covers the block's barrier on a and the fragment reads.
+// The four partial tiles are summed through LDS, in a's space, in group order.
+//
+// Eight K groups of one wave each (64 columns wide, a copied per wave) asked for a third more lines of
+// a where a wave's K range is no whole number of them (K = 768: 16 copies a row for 12 lines), left
+// eight partials to sum, and their LDS kept tiles at 64 rows, so that longer inputs ran two tiles a
+// CU or 128 x 128 tiles on half the CUs. Measured (MI355X, us a launch, that against this): 293 rows
+// qkv 5.67 / 5.15, wi 5.74 / 5.29, wo 4.01 / 3.86, wo_mlp 4.66 / 4.46; 400 rows qkv 6.37 / 5.68; 512
+// rows wi 9.64 / 6.66 (80-row tiles), wo_mlp 5.43 / 5.10; 650 rows qkv 9.97 / 7.20 (96-row tiles);
+// 1024 rows wo 5.90 / 5.48, wo_mlp 9.17 / 6.75. No gain: the fragments of every step read ahead of
+// the MFMAs (qkv 5.33), a group's two waves on one SIMD or adjacent (5.29).
+#pragma once
+
+#include <stdexcept>
+#include <string>
+
+#include "gemm_tile.h"
+
+namespace jh {
+
+// Dynamic LDS bytes for K: a's rows, or the four partials (rows padded to 68 floats) and a word for
+// the score's arrival.
+__host__ __device__ constexpr int group_lds_bytes(int bm, int k) {
+    return bm * k * 2 > 4 * bm * 68 * 4 + 16 ? bm * k * 2 : 4 * bm * 68 * 4 + 16;
+}
+constexpr int GROUP_LDS_MAX = 160 * 1024;
+
+// The K lines of the widest group (the instance that runs K), and the highest tile each instance has
+// (by a's LDS at its largest K).
+constexpr int group_lines(int k) { return (k >> 6) <= 8 ? 2 : ((k >> 6) + 3) / 4; }
+constexpr int group_rows_max(int kl) { return kl == 2 ? 128 : kl == 3 ? 96 : kl <= 5 ? 64 : kl == 6 ? 48 : 0; }
+
+// Task `task` of tiles_n * tiles_m (XCD-mapped); KL: the K lines of the widest group.
+template <int BM, int EPI, int KL>
+__device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, char* lds) {
+    constexpr int MI = BM / 16, RB = BM / 16;  // 16-row fragments; a wave's copies a line
+    constexpr int NPASS = (BM + 63) / 64;
+    const int L = xcd_task(task, p.tiles_n * p.tiles_m);
+    const int by = L % p.tiles_m, bx = L / p.tiles_m;
+    const int tid = threadIdx.x, l = tid & 63, r16 = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
+    const int kg = w & 3, ch = w >> 2;
+    const int NL = p.k >> 6, l0 = kg * NL >> 2, nl = ((kg + 1) * NL >> 2) - l0;  // KL or KL - 1 lines
+
+    // Copy (line, rb): rows 8 rb .. 8 rb + 7 of the line at LDS (line (BM / 8) + rb) 1024; lane l's 16
+    // bytes are row l / 8, chunk (l % 8) ^ sw(row), sw(r) = (r % 8) ^ ((r / 8) % 2): the 16 rows one
+    // fragment read takes cover the 64 banks.
+    uint32_t aoff[RB];
+    {
+        const int a_rows = (EPI & EPI_GATHER) ? p.src_m : p.m;
+        const auto ar = buffer_rsrc(p.a, (uint32_t)((size_t)a_rows * p.k * 2));
+#pragma unroll
+        for (int q = 0; q < RB; q++) {
+            const int r = 8 * (ch * RB + q) + (l >> 3);
+            const int row = min(by * BM + r, p.m - 1);  // rows past m: read, never stored
+            aoff[q] = ((uint32_t)src_row<EPI>(p, row) * (uint32_t)p.k +
+                       (uint32_t)(l0 * 64 + ((l & 7) ^ (r & 7) ^ ((r >> 3) & 1)) * 8)) * 2u;
+        }
+        char* dst = lds + (l0 * (BM / 8) + ch * RB) * 1024;
+#pragma unroll
+        for (int li = 0; li < KL; li++) {
+            if (li < KL - 1 || nl == KL) {  // (wave-uniform)
+#pragma unroll
+                for (int q = 0; q < RB; q++)
+                    lds_bdma16<false>(ar, aoff[q], dst + (li * (BM / 8) + q) * 1024, (uint32_t)li * 128u);
+            }
+        }
+    }
+
+    // The epilogue's other inputs, in flight with the operands.
+    const int c0 = (tid & 7) * 4;
+    EpiCol ec;
+    EpiRow er[NPASS];
+    epi_load_col<EPI>(p, bx, c0, ec);
+#pragma unroll
+    for (int ps = 0; ps < NPASS; ps++) epi_load_row<EPI, false>(p, by * BM + ps * 64 + (tid >> 3), bx, c0, er[ps]);
+
+    // w in fragment order: unit u's fragment j is 512 values at ((bx U + u) 4 + j) 512, lane l's 8 of
+    // them at 8 l. Through a descriptor over the group's units: a step past them reads zeros without
+    // touching memory.
+    half8 fw[2 * KL][2];
+    const auto wr = buffer_rsrc((const f16*)p.w + ((size_t)bx * 2 * NL + 2 * l0) * 2048, (uint32_t)nl * 8192);
+#pragma unroll
+    for (int s = 0; s < 2 * KL; s++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            fw[s][j] = bload16<false>(wr, (uint32_t)s * 4096 + (2 * ch + j) * 1024 + l * 16);
+#pragma unroll
+    for (int q = 0; q < RB; q++) asm volatile("" ::"v"(aoff[q]));  // (not w's registers: no wait for the copies)
+    __builtin_amdgcn_sched_barrier(0);
+    wait_vmcnt<4 * KL>();  // the copies, which went out before w's loads
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    // (The RoPE table rows wait for the positions: after the copies' wait, see gemm_tile.h.)
+#pragma unroll
+    for (int ps = 0; ps < NPASS; ps++) epi_load_rope<EPI>(p, by * BM + ps * 64 + (tid >> 3), c0, er[ps]);
+    __builtin_amdgcn_sched_barrier(0);
+
+    floatx4 acc[MI][2];
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int sw = (r16 & 7) ^ (r16 >> 3);
+    const char* ab = lds + l0 * (BM / 8) * 1024 + (r16 >> 3) * 1024 + (r16 & 7) * 128;
+#pragma unroll
+    for (int s = 0; s < 2 * KL; s++) {
+        if (s < 2 * KL - 2 || nl == KL) {  // (wave-uniform)
+            half8 fa[MI];
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+                fa[i] = *(const half8*)(ab + ((s >> 1) * (BM / 8) + 2 * i) * 1024 + 16 * ((4 * (s & 1) + g) ^ sw));
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) acc[i][j] = mfma16(fw[s][j], fa[i], acc[i][j]);
+        }
+    }
+    wait_lgkm0();
+    __builtin_amdgcn_s_barrier();  // every wave has read its rows of a: the partials take their space
+
+    // acc[i][j] lane: row 16 i + r16, columns 32 ch + 16 j + 4 g + e of the tile.
+    float* red = (float*)lds;  // [group][row][68]
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            *(floatx4*)&red[(kg * BM + 16 * i + r16) * 68 + 32 * ch + 16 * j + 4 * g] = acc[i][j];
+    __syncthreads();
+    float v[NPASS][8];
+#pragma unroll
+    for (int ps = 0; ps < NPASS; ps++) {
+        const int r = ps * 64 + (tid >> 3);
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[ps][e] = 0.0f;
+        if (r < BM) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float4 lo = *(const float4*)&red[(k * BM + r) * 68 + c0];
+                const float4 hi = *(const float4*)&red[(k * BM + r) * 68 + 32 + c0];
+                v[ps][0] += lo.x, v[ps][1] += lo.y, v[ps][2] += lo.z, v[ps][3] += lo.w;
+                v[ps][4] += hi.x, v[ps][5] += hi.y, v[ps][6] += hi.z, v[ps][7] += hi.w;
+            }
+        }
+    }
+    finish<NPASS, EPI, false, 512>(p, v, bx * p.tiles_m + by, 0, by * BM, bx, BM,
+                                 (uint32_t*)(lds + 4 * BM * 68 * 4), ec, er);
+}
+
+// ---- the kernel and its launcher, instantiated by the .hip files that include this -------------
+
+// Dynamic LDS: group_lds_bytes(BM, k), one block a CU.
+template <int BM, int EPI, int KL>
+__global__ __launch_bounds__(512, 1) void gemm_group(GemmParams p) {
+    extern __shared__ __attribute__((aligned(16))) char lds_dyn[];
+    gemm_group_tile<BM, EPI, KL>(p, blockIdx.x, lds_dyn);
+}
+
+template <int BM, int EPI, int KL>
+void launch_group(const GemmParams& p, hipStream_t st) {
+    static const bool lds_ok =  // once per instantiation, before its first launch
+        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_group<BM, EPI, KL>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, GROUP_LDS_MAX) == hipSuccess;
+    if (!lds_ok) throw std::runtime_error("gemm: the grouped latency kernel cannot have its LDS");
+    hipLaunchKernelGGL((gemm_group<BM, EPI, KL>), dim3(p.tiles_n * p.tiles_m), dim3(512), group_lds_bytes(BM, p.k),
+                       st, p);
+}
+
+template <int BM, int EPI, int KL = 2>
+void launch_group_lines(const GemmParams& p, hipStream_t st) {
+    if constexpr (BM <= group_rows_max(KL)) {
+        if (group_lines(p.k) == KL) launch_group<BM, EPI, KL>(p, st);
+        else launch_group_lines<BM, EPI, KL + 1>(p, st);
+    } else {
+        throw std::runtime_error("gemm: no grouped kernel for k = " + std::to_string(p.k));
+    }
+}
+
+template <int EPI>
+void launch_group_epi(const GemmParams& p, int bm, hipStream_t st) {
+    switch (bm) {
+        case 16: launch_group_lines<16, EPI>(p, st); break;
+        case 32: launch_group_lines<32, EPI>(p, st); break;
+        case 48: launch_group_lines<48, EPI>(p, st); break;
+        case 64: launch_group_lines<64, EPI>(p, st); break;
+        case 80: launch_group_lines<80, EPI>(p, st); break;
+        case 96: launch_group_lines<96, EPI>(p, st); break;
+        default: launch_group_lines<128, EPI>(p, st); break;
+    }
+}
+
+void gemm_group_launch_head(const GemmParams& p, int epi, int bm, hipStream_t st);
+
+}  // namespace jh

@@ -99,7 +99,8 @@ struct GemmConfig {
     int bm;      // rows per tile: 16, 32, 48, 64 (latency kernel), 128 (throughput kernel) or 192, 256
                  // (wide throughput kernel)
     int splits;  // K splits, 1-8
-    int height = 0;  // the wide kernel, unsplit: rows per tile (160, 192, 224, 256) in bm's place
+    int height = 0;  // unsplit, rows per tile in bm's place: with bm 256 the wide kernel's (160, 192,
+                     // 224, 256), with bm up to 64 the grouped latency kernel's (16 to 96, 128)
 };
 
 // Device scratch the split-K GEMMs and split-KV attention share (never at the same time).
@@ -136,6 +137,11 @@ struct Gemm {
 // The 256-column tiles of a checked GEMM, bm rows high (160, 192, 224 or 256; K splits 192 or 256).
 void gemm_wide_launch(const GemmParams& p, int epi, int bm, hipStream_t stream);
 int wide_height(int m, int n, int cus);
+// The grouped latency kernel: whether it takes tiles of bm rows at this k, the height it runs an
+// unsplit m x n x k GEMM with on `cus` CUs (0: it does not), and the launch of a checked GEMM.
+bool gemm_group_takes(int bm, int k);
+int gemm_group_height(int m, int n, int k, int cus);
+void gemm_group_launch(const GemmParams& p, int epi, int bm, hipStream_t stream);
 
 // Throws std::runtime_error when g or cfg break what the kernels assume.
 void gemm_check(const Gemm& g, GemmConfig cfg, const Scratch& s);
@@ -144,7 +150,8 @@ void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t st
 // (the throughput tiles only where they take the epilogue: LayerNorm up to k = GEMM_BIG_LN_MAX_K).
 GemmConfig gemm_choose(int m, int n, int k, int cus, int epi = 0);
 constexpr int GEMM_BIG_LN_MAX_K = 1024;
-// gemm_choose's pick as it is run: a throughput tile's kernel and height.
+// What a GEMM is run with: the grouped latency kernel or a throughput tile, with its height, in
+// place of gemm_choose's pick.
 GemmConfig gemm_pick(int m, int n, int k, int cus, int epi = 0);
 // Compute units of the current device (queried once per device; 256 if the query fails).
 int device_cus();

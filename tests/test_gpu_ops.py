@@ -168,15 +168,13 @@ def test_head_gemms(torch_cuda, scratch, kind, n, k):
     check_gemm(P, out, st, f"{kind} n={n} k={k}")
 
 
-# ---- the eight-wave latency kernel's K paths ----------------------------------------------
-# gemm_lat1 (grids of at most a block a CU) fixes its waves' K path per instance from K: wave w
-# of 8 takes K units [w U / 8, (w + 1) U / 8) of U = K / 32, all in one chunk when the busiest
-# wave has at most three (K <= 768), five (K <= 1280) or, on tiles of up to 32 rows, six
-# (K <= 1536) units, with a's lines staged through the wave's LDS slot, else in the chunked
-# loop. K at and around each boundary (320, 832 and 1344: waves whose range starts in the middle
-# of a 128-byte line; 1344 and 1536 on 48 and 64 rows, and 3072: the loop), every tile height,
-# M = 293 (rows past m in the last tile). Grids: 12 or 36 column tiles x 5-19 row tiles,
-# at most 252 blocks, so the eight-wave kernel runs on a 256-CU MI355X.
+# ---- the eight-wave latency kernels over K -------------------------------------------------
+# Grids of at most a block a CU: the grouped latency kernel cuts a's K / 64 lines of 128 bytes in
+# four groups, one instance per size of the widest (K up to 512, 768, 1024, 1280 and, on tiles of up
+# to 48 rows, 1536), a group having that many lines or one less; gemm_lat1 runs the rest. K at and
+# around each boundary (320, 832 and 1344: uneven groups; 1344 and 1536 on 64 rows, and 3072:
+# gemm_lat1), every tile height, M = 293 (rows past m in the last tile). Grids: 12 or 36 column
+# tiles x 5-19 row tiles, at most 252 blocks on a 256-CU MI355X.
 LAT1_KS = [256, 320, 768, 832, 1152, 1280, 1344, 1536, 3072]
 
 
@@ -189,6 +187,24 @@ def test_eight_wave_latency_tile_k_paths(torch_cuda, scratch, kind, n, bm, k):
     P = gemm_problem(kind, 293, n, k, seed=71 + k + bm)
     out, st = run_gemm(torch_cuda, P, bm, 1, scratch)
     check_gemm(P, out, st, f"{kind} n={n} k={k} bm={bm}")
+
+
+# The grouped latency kernel past 64 rows (bm 0: the pick on 256 CUs): 80, 96 and 128 rows at the
+# most K their instances take, uneven groups, a row short of a whole last tile or with one row in
+# it, 252 tiles; the tallest tiles of the longer K; one tile of one row.
+GROUP = [("lnrope", 559, 2304, 768), ("lngeglu", 560, 2304, 576), ("lnbias", 561, 2304, 704),
+         ("lnrope", 672, 2304, 768), ("resstats", 1921, 768, 640), ("lnbiasrelu", 2015, 768, 768),
+         ("lngeglu", 895, 2304, 512), ("biasresstats", 2561, 768, 256), ("lnbiasgelu", 2688, 768, 448),
+         ("resstats", 1343, 768, 1024), ("resstats", 1281, 768, 1280), ("biasresstats", 1007, 768, 1472),
+         ("lnbiasgelu", 1, 64, 256), ("resstats", 1, 64, 1536)]
+
+
+@pytest.mark.parametrize("kind,m,n,k", GROUP, ids=["-".join(map(str, g)) for g in GROUP])
+def test_grouped_latency_tile_heights(torch_cuda, scratch, kind, m, n, k):
+    say(f"grouped latency tiles {kind} M={m} N={n} K={k}")
+    P = gemm_problem(kind, m, n, k, seed=91 + m + k)
+    out, st = run_gemm(torch_cuda, P, 0, 1, scratch)
+    check_gemm(P, out, st, f"{kind} m={m} n={n} k={k}")
 
 
 # ---- MFMA-bound sizes ---------------------------------------------------------------------
