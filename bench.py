@@ -213,7 +213,11 @@ def gemm_instance(m, n, k, bm, epi, cus):
     top = {2: 128, 3: 96, 4: 64, 5: 64, 6: 48}.get(lines, 0) if k >= 256 else 0
     for h in (16, 32, 48, 64, 80, 96, 128):
         if h <= top and n // 64 * ceil(m, h) <= cus:
-            return f"gemm_group<{h}, {jh.EPI[epi]}, {lines}>"
+            return f"gemm_group<{h}, {jh.EPI[epi]}, {lines}, 1>"
+    low = {3: 64, 4: 48, 5: 48, 6: 32}.get(lines, 256)
+    for h in (32, 48, 64):
+        if n % 128 == 0 and low <= h <= top and not ("ln" in epi and k > 1024) and n // 128 * ceil(m, h) <= cus:
+            return f"gemm_group<{h}, {jh.EPI[epi]}, {lines}, 2>"
     if bm >= 128:  # the throughput kernel the launch takes (gemm_pick in csrc/gemm.hip)
         l128 = ceil(n // 128 * ceil(m, 128), cus)
         c128 = 2 + 8.5 * ks if l128 == 1 else 2.5 + 7.6 * ks * l128

@@ -389,6 +389,17 @@ __device__ __forceinline__ void epi_load_col(const GemmParams& p, int grp, int c
     }
 }
 
+// The residual of output row `row` (column group grp's columns c0, c0 + 32 and the three after each).
+template <int EPI, bool XR>
+__device__ __forceinline__ void epi_load_res(const GemmParams& p, int row, int grp, int c0, EpiRow& e) {
+    if ((EPI & EPI_RES) && !(EPI & EPI_GEGLU)) {
+        const int r = min(row, p.m - 1), rs = src_row<EPI>(p, r);
+        const f16* x = (const f16*)(p.res ? p.res : p.c) + (size_t)(p.res ? rs : r) * p.n + grp * 64 + c0;
+        e.rl = load8h<XR>(x);
+        e.rh = load8h<XR>(x + 32);
+    }
+}
+
 // XS: the statistics are read device-coherent; XR: the residual rows are.
 template <int EPI, bool XS, bool XR = XS>
 __device__ __forceinline__ void epi_load_row(const GemmParams& p, int row, int grp, int c0,
@@ -407,11 +418,7 @@ __device__ __forceinline__ void epi_load_row(const GemmParams& p, int row, int g
         // The choice between it and the row waits for the load: epi_load_rope makes it.
         e.pos = *(const int*)(p.pos ? (const void*)(p.pos + r) : (const void*)p.rope);
     }
-    if ((EPI & EPI_RES) && !(EPI & EPI_GEGLU)) {
-        const f16* x = (const f16*)(p.res ? p.res : p.c) + (size_t)(p.res ? rs : r) * p.n + grp * 64 + c0;
-        e.rl = load8h<XR>(x);
-        e.rh = load8h<XR>(x + 32);
-    }
+    epi_load_res<EPI, XR>(p, row, grp, c0, e);
 }
 
 // The RoPE table row of output row `row`'s position (e.pos, loaded by epi_load_row): a separate

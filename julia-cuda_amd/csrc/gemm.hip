@@ -3,7 +3,7 @@
 // kernels/src/main.rs:886-1041) walks K through shared tiles with 4-8 warps each owning a
 // piece of the output; here two kernels cover the two regimes of a 256-CU GPU:
 //
-//  - gemm_group (16 to 128 rows x 64 columns, gemm_group.h): the latency-bound regime, grids of at
+//  - gemm_group (16 to 128 rows x 64 columns, 32 to 64 x 128, gemm_group.h): the latency-bound regime, grids of at
 //    most a block a CU (every GEMM of a request of up to 672 tokens): eight waves in four K groups,
 //    a's rows whole in LDS, w straight into registers, the partial tiles summed through LDS.
 //  - gemm_lat (BM = 16/32/48/64 rows x 64 columns): more tiles than CUs, or a K split. The block's
@@ -251,6 +251,7 @@ void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t st
     const bool group = cfg.bm < 128 && cfg.splits == 1 && gemm_group_takes(bm, g.k) &&
                        (cfg.height || p.tiles_n * p.tiles_m <= device_cus());
     if (group) gemm_group_launch(p, g.epi, bm, st);
+    else if (cfg.bm == 128 && cfg.height) gemm_group2_launch(p, g.epi, bm, st);
     else switch (g.epi) {
         case EPI_K_ROPE: launch_epi<EPI_K_ROPE>(p, bm, st); break;
         case EPI_K_LNROPE: launch_epi<EPI_K_LNROPE>(p, bm, st); break;
@@ -407,10 +408,12 @@ GemmConfig gemm_choose(int m, int n, int k, int cus, int epi) {
 // for the wide tiles; wo_mlp level, 23.5), the wide tiles for qkv and wi from 4096 (18.5 us
 // against 25) and for everything at 18752.
 // And before these, wherever a grid of at most a block a CU covers the GEMM, the grouped latency
-// kernel at its smallest such height (gemm_group.hip has the figures).
+// kernel at its smallest such height, on 64 columns or else on 128 (gemm_group.hip and gemm_group2.hip
+// have the figures).
 GemmConfig gemm_pick(int m, int n, int k, int cus, int epi) {
     if (cus <= 0) cus = 256;
     if (const int h = gemm_group_height(m, n, k, cus)) return GemmConfig{std::min(h, 64), 1, h};
+    if (const int h = gemm_group2_height(m, n, k, cus, epi)) return GemmConfig{128, 1, h};
     GemmConfig best = gemm_choose(m, n, k, cus, epi);
     if (best.bm < 128) return best;
     const double ks = (double)k / 768.0;

@@ -1,5 +1,5 @@
-// One output tile of the grouped latency GEMM (BM rows x 64 columns), for grids of at most a block a
-// CU: eight waves in four K groups of two column halves.
+// One output tile of the grouped latency GEMM (BM rows x 64 columns, or 128), for grids of at most a
+// block a CU: eight waves in four K groups of two column halves.
 //
 // Bound by a launch and a first round trip (~2.5 us), then by how fast a CU takes in its operands: a
 // 48-row tile at K = 768 asks for 1344 lines of 128 bytes, about 2 ns each.
@@ -39,11 +39,17 @@ constexpr int GROUP_LDS_MAX = 160 * 1024;
 // (by a's LDS at its largest K).
 constexpr int group_lines(int k) { return (k >> 6) <= 8 ? 2 : ((k >> 6) + 3) / 4; }
 constexpr int group_rows_max(int kl) { return kl == 2 ? 128 : kl == 3 ? 96 : kl <= 5 ? 64 : kl == 6 ? 48 : 0; }
+// The lowest tile of 128 columns: past what the highest of 64 columns covers.
+constexpr int group2_rows_min(int kl) { return kl == 2 ? 256 : kl == 3 ? 64 : kl <= 5 ? 48 : 32; }
+constexpr int GROUP2_ROWS_MAX = 64;  // (past it the sum and the epilogue take what the K loop gains)
 
-// Task `task` of tiles_n * tiles_m (XCD-mapped); KL: the K lines of the widest group.
-template <int BM, int EPI, int KL>
+// Task `task` of tiles_n * tiles_m (XCD-mapped); KL: the K lines of the widest group; NC: the tile's
+// 64-column groups.
+template <int BM, int EPI, int KL, int NC>
 __device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, char* lds) {
     constexpr int MI = BM / 16, RB = BM / 16;  // 16-row fragments; a wave's copies a line
+    constexpr int FJ = 2 * NC;                 // a wave's 16-column fragments
+    constexpr int D = NC == 1 || 2 * KL < 6 ? 2 * KL : 6;  // K steps of w in flight
     constexpr int NPASS = (BM + 63) / 64;
     const int L = xcd_task(task, p.tiles_n * p.tiles_m);
     const int by = L % p.tiles_m, bx = L / p.tiles_m;
@@ -81,24 +87,27 @@ __device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, c
     const int c0 = (tid & 7) * 4;
     EpiCol ec;
     EpiRow er[NPASS];
-    epi_load_col<EPI>(p, bx, c0, ec);
+    epi_load_col<EPI>(p, NC * bx, c0, ec);
 #pragma unroll
-    for (int ps = 0; ps < NPASS; ps++) epi_load_row<EPI, false>(p, by * BM + ps * 64 + (tid >> 3), bx, c0, er[ps]);
+    for (int ps = 0; ps < NPASS; ps++) epi_load_row<EPI, false>(p, by * BM + ps * 64 + (tid >> 3), NC * bx, c0, er[ps]);
 
-    // w in fragment order: unit u's fragment j is 512 values at ((bx U + u) 4 + j) 512, lane l's 8 of
-    // them at 8 l. Through a descriptor over the group's units: a step past them reads zeros without
-    // touching memory.
-    half8 fw[2 * KL][2];
-    const auto wr = buffer_rsrc((const f16*)p.w + ((size_t)bx * 2 * NL + 2 * l0) * 2048, (uint32_t)nl * 8192);
+    // w in fragment order: unit u's fragment j of column group c is 512 values at ((c U + u) 4 + j) 512,
+    // lane l's 8 of them at 8 l. Through a descriptor over the group's units: a step past them reads
+    // zeros without touching memory.
+    half8 fw[D][FJ];
+    const int wg = NC == 1 ? bx : 2 * bx + ch, j0 = NC == 1 ? 2 * ch : 0;
+    const auto wr = buffer_rsrc((const f16*)p.w + ((size_t)wg * 2 * NL + 2 * l0) * 2048, (uint32_t)nl * 8192);
+    auto load_w = [&](int s) {
 #pragma unroll
-    for (int s = 0; s < 2 * KL; s++)
+        for (int j = 0; j < FJ; j++)
+            fw[s % D][j] = bload16<false>(wr, (uint32_t)s * 4096 + (j0 + j) * 1024 + l * 16);
+    };
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-            fw[s][j] = bload16<false>(wr, (uint32_t)s * 4096 + (2 * ch + j) * 1024 + l * 16);
+    for (int s = 0; s < D; s++) load_w(s);
 #pragma unroll
     for (int q = 0; q < RB; q++) asm volatile("" ::"v"(aoff[q]));  // (not w's registers: no wait for the copies)
     __builtin_amdgcn_sched_barrier(0);
-    wait_vmcnt<4 * KL>();  // the copies, which went out before w's loads
+    wait_vmcnt<D * FJ>();  // the copies, which went out before w's loads
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     // (The RoPE table rows wait for the positions: after the copies' wait, see gemm_tile.h.)
@@ -106,11 +115,11 @@ __device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, c
     for (int ps = 0; ps < NPASS; ps++) epi_load_rope<EPI>(p, by * BM + ps * 64 + (tid >> 3), c0, er[ps]);
     __builtin_amdgcn_sched_barrier(0);
 
-    floatx4 acc[MI][2];
+    floatx4 acc[MI][FJ];
 #pragma unroll
     for (int i = 0; i < MI; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < FJ; j++) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     const int sw = (r16 & 7) ^ (r16 >> 3);
     const char* ab = lds + l0 * (BM / 8) * 1024 + (r16 >> 3) * 1024 + (r16 & 7) * 128;
 #pragma unroll
@@ -123,64 +132,85 @@ __device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, c
 #pragma unroll
             for (int i = 0; i < MI; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = mfma16(fw[s][j], fa[i], acc[i][j]);
+                for (int j = 0; j < FJ; j++) acc[i][j] = mfma16(fw[s % D][j], fa[i], acc[i][j]);
+        }
+        if (s + D < 2 * KL) load_w(s + D);
+    }
+    EpiCol ec1;  // the second column group's inputs
+    EpiRow er1[NPASS];
+    if constexpr (NC == 2) {
+        epi_load_col<EPI>(p, 2 * bx + 1, c0, ec1);
+#pragma unroll
+        for (int ps = 0; ps < NPASS; ps++) {
+            er1[ps] = er[ps];
+            epi_load_res<EPI, false>(p, by * BM + ps * 64 + (tid >> 3), 2 * bx + 1, c0, er1[ps]);
         }
     }
     wait_lgkm0();
     __builtin_amdgcn_s_barrier();  // every wave has read its rows of a: the partials take their space
 
-    // acc[i][j] lane: row 16 i + r16, columns 32 ch + 16 j + 4 g + e of the tile.
-    float* red = (float*)lds;  // [group][row][68]
+    // acc[i][j] lane: row 16 i + r16, columns 16 (j0 + j) + 4 g + e of its column group. The groups one
+    // after the other: partials, sum, epilogue.
+    float* red = (float*)lds;  // [K group][row][68]
 #pragma unroll
-    for (int i = 0; i < MI; i++)
+    for (int cg = 0; cg < NC; cg++) {
+        if (NC == 1 || ch == cg) {
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-            *(floatx4*)&red[(kg * BM + 16 * i + r16) * 68 + 32 * ch + 16 * j + 4 * g] = acc[i][j];
-    __syncthreads();
-    float v[NPASS][8];
+            for (int i = 0; i < MI; i++)
 #pragma unroll
-    for (int ps = 0; ps < NPASS; ps++) {
-        const int r = ps * 64 + (tid >> 3);
+                for (int j = 0; j < FJ; j++)
+                    *(floatx4*)&red[(kg * BM + 16 * i + r16) * 68 + 16 * (j0 + j) + 4 * g] = acc[i][j];
+        }
+        __syncthreads();
+        float v[NPASS][8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[ps][e] = 0.0f;
-        if (r < BM) {
+        for (int ps = 0; ps < NPASS; ps++) {
+            const int r = ps * 64 + (tid >> 3);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const float4 lo = *(const float4*)&red[(k * BM + r) * 68 + c0];
-                const float4 hi = *(const float4*)&red[(k * BM + r) * 68 + 32 + c0];
-                v[ps][0] += lo.x, v[ps][1] += lo.y, v[ps][2] += lo.z, v[ps][3] += lo.w;
-                v[ps][4] += hi.x, v[ps][5] += hi.y, v[ps][6] += hi.z, v[ps][7] += hi.w;
+            for (int e = 0; e < 8; e++) v[ps][e] = 0.0f;
+            if (r < BM) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float4 lo = *(const float4*)&red[(k * BM + r) * 68 + c0];
+                    const float4 hi = *(const float4*)&red[(k * BM + r) * 68 + 32 + c0];
+                    v[ps][0] += lo.x, v[ps][1] += lo.y, v[ps][2] += lo.z, v[ps][3] += lo.w;
+                    v[ps][4] += hi.x, v[ps][5] += hi.y, v[ps][6] += hi.z, v[ps][7] += hi.w;
+                }
             }
         }
+        if (cg + 1 < NC) __syncthreads();
+        finish<NPASS, EPI, false, 512>(p, v, bx * p.tiles_m + by, 0, by * BM, NC * bx + cg, BM,
+                                       (uint32_t*)(lds + 4 * BM * 68 * 4), cg ? ec1 : ec, cg ? er1 : er);
     }
-    finish<NPASS, EPI, false, 512>(p, v, bx * p.tiles_m + by, 0, by * BM, bx, BM,
-                                 (uint32_t*)(lds + 4 * BM * 68 * 4), ec, er);
 }
 
 // ---- the kernel and its launcher, instantiated by the .hip files that include this -------------
 
 // Dynamic LDS: group_lds_bytes(BM, k), one block a CU.
-template <int BM, int EPI, int KL>
+template <int BM, int EPI, int KL, int NC>
 __global__ __launch_bounds__(512, 1) void gemm_group(GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) char lds_dyn[];
-    gemm_group_tile<BM, EPI, KL>(p, blockIdx.x, lds_dyn);
+    gemm_group_tile<BM, EPI, KL, NC>(p, blockIdx.x, lds_dyn);
 }
 
-template <int BM, int EPI, int KL>
+template <int BM, int EPI, int KL, int NC>
 void launch_group(const GemmParams& p, hipStream_t st) {
     static const bool lds_ok =  // once per instantiation, before its first launch
-        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_group<BM, EPI, KL>),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_group<BM, EPI, KL, NC>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, GROUP_LDS_MAX) == hipSuccess;
     if (!lds_ok) throw std::runtime_error("gemm: the grouped latency kernel cannot have its LDS");
-    hipLaunchKernelGGL((gemm_group<BM, EPI, KL>), dim3(p.tiles_n * p.tiles_m), dim3(512), group_lds_bytes(BM, p.k),
+    hipLaunchKernelGGL((gemm_group<BM, EPI, KL, NC>), dim3(p.tiles_n * p.tiles_m), dim3(512), group_lds_bytes(BM, p.k),
                        st, p);
 }
 
-template <int BM, int EPI, int KL = 2>
+template <int BM, int EPI, int NC, int KL = 2>
 void launch_group_lines(const GemmParams& p, hipStream_t st) {
-    if constexpr (BM <= group_rows_max(KL)) {
-        if (group_lines(p.k) == KL) launch_group<BM, EPI, KL>(p, st);
-        else launch_group_lines<BM, EPI, KL + 1>(p, st);
+    if constexpr (NC == 2 && BM < group2_rows_min(KL)) {
+        if (group_lines(p.k) != KL) launch_group_lines<BM, EPI, NC, KL + 1>(p, st);
+        else throw std::runtime_error("gemm: no grouped kernel for k = " + std::to_string(p.k));
+    } else if constexpr (BM <= group_rows_max(KL)) {
+        if (group_lines(p.k) == KL) launch_group<BM, EPI, KL, NC>(p, st);
+        else launch_group_lines<BM, EPI, NC, KL + 1>(p, st);
     } else {
         throw std::runtime_error("gemm: no grouped kernel for k = " + std::to_string(p.k));
     }
@@ -189,13 +219,22 @@ void launch_group_lines(const GemmParams& p, hipStream_t st) {
 template <int EPI>
 void launch_group_epi(const GemmParams& p, int bm, hipStream_t st) {
     switch (bm) {
-        case 16: launch_group_lines<16, EPI>(p, st); break;
-        case 32: launch_group_lines<32, EPI>(p, st); break;
-        case 48: launch_group_lines<48, EPI>(p, st); break;
-        case 64: launch_group_lines<64, EPI>(p, st); break;
-        case 80: launch_group_lines<80, EPI>(p, st); break;
-        case 96: launch_group_lines<96, EPI>(p, st); break;
-        default: launch_group_lines<128, EPI>(p, st); break;
+        case 16: launch_group_lines<16, EPI, 1>(p, st); break;
+        case 32: launch_group_lines<32, EPI, 1>(p, st); break;
+        case 48: launch_group_lines<48, EPI, 1>(p, st); break;
+        case 64: launch_group_lines<64, EPI, 1>(p, st); break;
+        case 80: launch_group_lines<80, EPI, 1>(p, st); break;
+        case 96: launch_group_lines<96, EPI, 1>(p, st); break;
+        default: launch_group_lines<128, EPI, 1>(p, st); break;
+    }
+}
+
+template <int EPI>
+void launch_group2_epi(const GemmParams& p, int bm, hipStream_t st) {
+    switch (bm) {
+        case 32: launch_group_lines<32, EPI, 2>(p, st); break;
+        case 48: launch_group_lines<48, EPI, 2>(p, st); break;
+        default: launch_group_lines<64, EPI, 2>(p, st); break;
     }
 }
 

@@ -1,0 +1,39 @@
+// The grouped latency GEMM (gemm_group.h) on tiles two column groups wide.
+#include "gemm_group.h"
+
+namespace jh {
+
+static bool group2_takes(int bm, int k) {
+    const int kl = group_lines(k);
+    return k >= 256 && bm >= group2_rows_min(kl) && bm <= group_rows_max(kl) && bm <= GROUP2_ROWS_MAX &&
+           group_lds_bytes(bm, k) <= GROUP_LDS_MAX;
+}
+
+// The smallest such tile whose grid is at most a block a CU (0: none), where gemm_group_height has
+// none. Against 128 x 128 tiles on part of the CUs (MI355X, us, those / this): qkv at 896 rows 10.3 /
+// 8.4 on 64-row tiles, wo at 2048 and 2600 rows 9.4 / 7.9 and 9.6 / 8.1; wo_mlp (K = 1152) at 1500
+// rows 12.8 / 8.8 on 48-row tiles, at 2048 and 2600 rows 15.9 / 10.5 and 16.7 / 13.0 on 64. 80- and
+// 96-row tiles were level or slower (qkv at 1024 rows 10.3 / 10.0 / 10.7), as was every one at K = 384.
+int gemm_group2_height(int m, int n, int k, int cus, int epi) {
+    if (n % 128 || (epi & (EPI_GATHER | EPI_SCORE)) || ((epi & EPI_LN) && k > GEMM_BIG_LN_MAX_K)) return 0;
+    for (int h : {32, 48, 64})
+        if (group2_takes(h, k) && (long)(n / 128) * (((long)m + h - 1) / h) <= cus) return h;
+    return 0;
+}
+
+void gemm_group2_launch(const GemmParams& p, int epi, int bm, hipStream_t st) {
+    switch (epi) {
+        case EPI_K_ROPE: launch_group2_epi<EPI_K_ROPE>(p, bm, st); break;
+        case EPI_K_LNROPE: launch_group2_epi<EPI_K_LNROPE>(p, bm, st); break;
+        case EPI_K_LNGEGLU: launch_group2_epi<EPI_K_LNGEGLU>(p, bm, st); break;
+        case EPI_K_RESSTATS: launch_group2_epi<EPI_K_RESSTATS>(p, bm, st); break;
+        case EPI_K_LNBIAS: launch_group2_epi<EPI_K_LNBIAS>(p, bm, st); break;
+        case EPI_K_LNBIASRELU: launch_group2_epi<EPI_K_LNBIASRELU>(p, bm, st); break;
+        case EPI_K_LNBIASGELU: launch_group2_epi<EPI_K_LNBIASGELU>(p, bm, st); break;
+        case EPI_K_BIASRESSTATS: launch_group2_epi<EPI_K_BIASRESSTATS>(p, bm, st); break;
+        case 0: launch_group2_epi<0>(p, bm, st); break;
+        default: throw std::runtime_error("gemm: no two-group kernel for epilogue " + std::to_string(epi));
+    }
+}
+
+}  // namespace jh

@@ -100,7 +100,8 @@ struct GemmConfig {
                  // (wide throughput kernel)
     int splits;  // K splits, 1-8
     int height = 0;  // unsplit, rows per tile in bm's place: with bm 256 the wide kernel's (160, 192,
-                     // 224, 256), with bm up to 64 the grouped latency kernel's (16 to 96, 128)
+                     // 224, 256), with bm up to 64 the grouped latency kernel's (16 to 96, 128), with bm
+                     // 128 that kernel's on 128 columns (32, 48, 64)
 };
 
 // Device scratch the split-K GEMMs and split-KV attention share (never at the same time).
@@ -142,6 +143,9 @@ int wide_height(int m, int n, int cus);
 bool gemm_group_takes(int bm, int k);
 int gemm_group_height(int m, int n, int k, int cus);
 void gemm_group_launch(const GemmParams& p, int epi, int bm, hipStream_t stream);
+// The same on tiles of 128 columns.
+int gemm_group2_height(int m, int n, int k, int cus, int epi);
+void gemm_group2_launch(const GemmParams& p, int epi, int bm, hipStream_t stream);
 
 // Throws std::runtime_error when g or cfg break what the kernels assume.
 void gemm_check(const Gemm& g, GemmConfig cfg, const Scratch& s);

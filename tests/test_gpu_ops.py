@@ -196,7 +196,11 @@ GROUP = [("lnrope", 559, 2304, 768), ("lngeglu", 560, 2304, 576), ("lnbias", 561
          ("lnrope", 672, 2304, 768), ("resstats", 1921, 768, 640), ("lnbiasrelu", 2015, 768, 768),
          ("lngeglu", 895, 2304, 512), ("biasresstats", 2561, 768, 256), ("lnbiasgelu", 2688, 768, 448),
          ("resstats", 1343, 768, 1024), ("resstats", 1281, 768, 1280), ("biasresstats", 1007, 768, 1472),
-         ("lnbiasgelu", 1, 64, 256), ("resstats", 1, 64, 1536)]
+         ("lnbiasgelu", 1, 64, 256), ("resstats", 1, 64, 1536),
+         # two column groups: 64 rows (three lines), 48 and 64 (four and five), 32 and 48 (six)
+         ("lnrope", 673, 2304, 768), ("lngeglu", 895, 2304, 576), ("biasresstats", 2688, 768, 704),
+         ("lnbias", 449, 2304, 832), ("lnbiasrelu", 2625, 768, 1024), ("resstats", 1345, 768, 1152),
+         ("biasresstats", 2687, 768, 1280), ("resstats", 1009, 768, 1536), ("resstats", 2015, 768, 1344)]
 
 
 @pytest.mark.parametrize("kind,m,n,k", GROUP, ids=["-".join(map(str, g)) for g in GROUP])
