@@ -211,6 +211,8 @@ def gemm_instance(m, n, k, bm, epi, cus):
     ks, ceil = k / 768, lambda a, b: -(-a // b)
     lines = max(2, ceil(k // 64, 4))  # the grouped latency kernel's instance and its highest tile
     top = {2: 128, 3: 96, 4: 64, 5: 64, 6: 48}.get(lines, 0) if k >= 256 else 0
+    if top and not ("stats" in epi or "score" in epi) and n // 32 * ceil(m, 16) <= cus:
+        return f"gemm_group<16, {jh.EPI[epi]}, {lines}, 0>"
     for h in (16, 32, 48, 64, 80, 96, 128):
         if h <= top and n // 64 * ceil(m, h) <= cus:
             return f"gemm_group<{h}, {jh.EPI[epi]}, {lines}, 1>"

@@ -3,7 +3,8 @@
 // kernels/src/main.rs:886-1041) walks K through shared tiles with 4-8 warps each owning a
 // piece of the output; here two kernels cover the two regimes of a 256-CU GPU:
 //
-//  - gemm_group (16 to 128 rows x 64 columns, 32 to 64 x 128, gemm_group.h): the latency-bound regime, grids of at
+//  - gemm_group (16 to 128 rows x 64 columns, 32 to 64 x 128, 16 x 32,
+//    gemm_group.h): the latency-bound regime, grids of at
 //    most a block a CU (every GEMM of a request of up to 672 tokens): eight waves in four K groups,
 //    a's rows whole in LDS, w straight into registers, the partial tiles summed through LDS.
 //  - gemm_lat (BM = 16/32/48/64 rows x 64 columns): more tiles than CUs, or a K split. The block's
@@ -250,7 +251,10 @@ void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t st
     p.tiles_m = (g.m + bm - 1) / bm;
     const bool group = cfg.bm < 128 && cfg.splits == 1 && gemm_group_takes(bm, g.k) &&
                        (cfg.height || p.tiles_n * p.tiles_m <= device_cus());
-    if (group) gemm_group_launch(p, g.epi, bm, st);
+    if (group && bm == 16 && gemm_group0_takes(g.m, g.n, g.k, device_cus(), g.epi)) {
+        p.tiles_n = g.n / 32;
+        gemm_group0_launch(p, g.epi, st);
+    } else if (group) gemm_group_launch(p, g.epi, bm, st);
     else if (cfg.bm == 128 && cfg.height) gemm_group2_launch(p, g.epi, bm, st);
     else switch (g.epi) {
         case EPI_K_ROPE: launch_epi<EPI_K_ROPE>(p, bm, st); break;

@@ -1,4 +1,4 @@
-// One output tile of the grouped latency GEMM (BM rows x 64 columns, or 128), for grids of at most a
+// One output tile of the grouped latency GEMM (BM rows x 64 columns, or 128, or 32), for grids of at most a
 // block a CU: eight waves in four K groups of two column halves.
 //
 // Bound by a launch and a first round trip (~2.5 us), then by how fast a CU takes in its operands: a
@@ -44,15 +44,19 @@ constexpr int group2_rows_min(int kl) { return kl == 2 ? 256 : kl == 3 ? 64 : kl
 constexpr int GROUP2_ROWS_MAX = 64;  // (past it the sum and the epilogue take what the K loop gains)
 
 // Task `task` of tiles_n * tiles_m (XCD-mapped); KL: the K lines of the widest group; NC: the tile's
-// 64-column groups.
+// 64-column groups, 0: half of one, columns 16 h .. + 15 and 32 + 16 h .. + 15 (the RoPE and GeGLU pairs
+// x, x + 32 whole; not the statistics of a group's output, nor the score's partials).
 template <int BM, int EPI, int KL, int NC>
 __device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, char* lds) {
     constexpr int MI = BM / 16, RB = BM / 16;  // 16-row fragments; a wave's copies a line
-    constexpr int FJ = 2 * NC;                 // a wave's 16-column fragments
-    constexpr int D = NC == 1 || 2 * KL < 6 ? 2 * KL : 6;  // K steps of w in flight
+    constexpr int FJ = NC ? 2 * NC : 1;        // a wave's 16-column fragments
+    constexpr int CG = NC ? NC : 1;            // the tile's column groups, whole or in part
+    static_assert(NC || !(EPI & (EPI_STATS | EPI_SCORE)), "half a column group");
+    constexpr int D = NC <= 1 || 2 * KL < 6 ? 2 * KL : 6;  // K steps of w in flight
     constexpr int NPASS = (BM + 63) / 64;
     const int L = xcd_task(task, p.tiles_n * p.tiles_m);
-    const int by = L % p.tiles_m, bx = L / p.tiles_m;
+    const int by = L % p.tiles_m, bt = L / p.tiles_m;
+    const int bx = NC ? bt : bt >> 1, hb = bt & 1;  // (hb: the half, with NC = 0)
     const int tid = threadIdx.x, l = tid & 63, r16 = l & 15, g = l >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
     const int kg = w & 3, ch = w >> 2;
@@ -87,15 +91,15 @@ __device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, c
     const int c0 = (tid & 7) * 4;
     EpiCol ec;
     EpiRow er[NPASS];
-    epi_load_col<EPI>(p, NC * bx, c0, ec);
+    epi_load_col<EPI>(p, CG * bx, c0, ec);
 #pragma unroll
-    for (int ps = 0; ps < NPASS; ps++) epi_load_row<EPI, false>(p, by * BM + ps * 64 + (tid >> 3), NC * bx, c0, er[ps]);
+    for (int ps = 0; ps < NPASS; ps++) epi_load_row<EPI, false>(p, by * BM + ps * 64 + (tid >> 3), CG * bx, c0, er[ps]);
 
     // w in fragment order: unit u's fragment j of column group c is 512 values at ((c U + u) 4 + j) 512,
     // lane l's 8 of them at 8 l. Through a descriptor over the group's units: a step past them reads
     // zeros without touching memory.
     half8 fw[D][FJ];
-    const int wg = NC == 1 ? bx : 2 * bx + ch, j0 = NC == 1 ? 2 * ch : 0;
+    const int wg = NC == 2 ? 2 * bx + ch : bx, j0 = NC == 2 ? 0 : NC == 1 ? 2 * ch : hb + 2 * ch;
     const auto wr = buffer_rsrc((const f16*)p.w + ((size_t)wg * 2 * NL + 2 * l0) * 2048, (uint32_t)nl * 8192);
     auto load_w = [&](int s) {
 #pragma unroll
@@ -153,8 +157,8 @@ __device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, c
     // after the other: partials, sum, epilogue.
     float* red = (float*)lds;  // [K group][row][68]
 #pragma unroll
-    for (int cg = 0; cg < NC; cg++) {
-        if (NC == 1 || ch == cg) {
+    for (int cg = 0; cg < CG; cg++) {
+        if (CG == 1 || ch == cg) {
 #pragma unroll
             for (int i = 0; i < MI; i++)
 #pragma unroll
@@ -178,9 +182,10 @@ __device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, c
                 }
             }
         }
-        if (cg + 1 < NC) __syncthreads();
-        finish<NPASS, EPI, false, 512>(p, v, bx * p.tiles_m + by, 0, by * BM, NC * bx + cg, BM,
-                                       (uint32_t*)(lds + 4 * BM * 68 * 4), cg ? ec1 : ec, cg ? er1 : er);
+        if (cg + 1 < CG) __syncthreads();
+        finish<NPASS, EPI, false, 512>(p, v, bx * p.tiles_m + by, 0, by * BM, CG * bx + cg, BM,
+                                       (uint32_t*)(lds + 4 * BM * 68 * 4), cg ? ec1 : ec, cg ? er1 : er,
+                                       NC || (c0 >> 4) == hb);
     }
 }
 
@@ -236,6 +241,11 @@ void launch_group2_epi(const GemmParams& p, int bm, hipStream_t st) {
         case 48: launch_group_lines<48, EPI, 2>(p, st); break;
         default: launch_group_lines<64, EPI, 2>(p, st); break;
     }
+}
+
+template <int EPI>
+void launch_group0_epi(const GemmParams& p, hipStream_t st) {
+    launch_group_lines<16, EPI, 0>(p, st);
 }
 
 void gemm_group_launch_head(const GemmParams& p, int epi, int bm, hipStream_t st);

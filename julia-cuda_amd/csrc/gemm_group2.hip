@@ -1,4 +1,4 @@
-// The grouped latency GEMM (gemm_group.h) on tiles two column groups wide.
+// The grouped latency GEMM (gemm_group.h) on tiles of two column groups, and of half a one.
 #include "gemm_group.h"
 
 namespace jh {
@@ -19,6 +19,27 @@ int gemm_group2_height(int m, int n, int k, int cus, int epi) {
     for (int h : {32, 48, 64})
         if (group2_takes(h, k) && (long)(n / 128) * (((long)m + h - 1) / h) <= cus) return h;
     return 0;
+}
+
+// Tiles of 16 rows x 32 columns where that grid is at most a block a CU: a CU then takes in half of
+// w's 64 columns (MI355X, us, 16 x 64 tiles / this: the scorer's lin1 on 6 rows 4.1 / 3.6, linear1 on 80
+// rows 3.9 / 3.5, qkv on 48 rows 3.95 / 3.4, at d = 384 on 100 rows 4.0 / 3.2). Not with output statistics (a group's are one block's) or the score.
+bool gemm_group0_takes(int m, int n, int k, int cus, int epi) {
+    return k >= 256 && group_rows_max(group_lines(k)) && !(epi & (EPI_STATS | EPI_SCORE | EPI_GATHER)) &&
+           (long)(n / 32) * (((long)m + 15) / 16) <= cus;
+}
+
+void gemm_group0_launch(const GemmParams& p, int epi, hipStream_t st) {
+    switch (epi) {
+        case EPI_K_ROPE: launch_group0_epi<EPI_K_ROPE>(p, st); break;
+        case EPI_K_LNROPE: launch_group0_epi<EPI_K_LNROPE>(p, st); break;
+        case EPI_K_LNGEGLU: launch_group0_epi<EPI_K_LNGEGLU>(p, st); break;
+        case EPI_K_LNBIAS: launch_group0_epi<EPI_K_LNBIAS>(p, st); break;
+        case EPI_K_LNBIASRELU: launch_group0_epi<EPI_K_LNBIASRELU>(p, st); break;
+        case EPI_K_LNBIASGELU: launch_group0_epi<EPI_K_LNBIASGELU>(p, st); break;
+        case 0: launch_group0_epi<0>(p, st); break;
+        default: throw std::runtime_error("gemm: no half-group kernel for epilogue " + std::to_string(epi));
+    }
 }
 
 void gemm_group2_launch(const GemmParams& p, int epi, int bm, hipStream_t st) {

@@ -26,6 +26,8 @@ constexpr int LAT_SPLIT_PASS_ROWS = 32;
 // reduction when the grid splits K -> the epilogue. Thread t of NT owns row (pass * NT / 8 +
 // t / 8) of the tile and columns c0 = 4 (t % 8), c0 + 32 of 64-column group `grp`.
 //
+// cols: whether the thread's columns are the tile's (the grouped kernel's tiles of half a group).
+//
 // Split-K (kernels/src/gemm.rs:355-433): every block writes its partial to the scratch
 // (device-coherent stores), waits for them to complete, then counts its arrival; the last of the
 // tile's splits (which resets the counter) invalidates its caches and sums all partials in split
@@ -34,7 +36,7 @@ template <int NPASS, int EPI, bool XG = false, int NT = 256>
 __device__ __forceinline__ void finish(const GemmParams& p, float (&v)[NPASS][8], int tile_id,
                                        int z, int row0, int grp, int rows_in_tile,
                                        uint32_t* s_last, const EpiCol& ec,
-                                       const EpiRow (&er)[NPASS]) {
+                                       const EpiRow (&er)[NPASS], bool cols = true) {
     const int tid = threadIdx.x;
     if (p.splits > 1) {
         // [tile][split][pass][half][thread] float4s: coalesced stores and loads.
@@ -83,7 +85,7 @@ __device__ __forceinline__ void finish(const GemmParams& p, float (&v)[NPASS][8]
     for (int ps = 0; ps < NPASS; ps++) {
         const int r = ps * (NT / 8) + (tid >> 3);
         const int row = row0 + r;
-        epi_apply<EPI, XG>(p, row, grp, c0, v[ps], r < rows_in_tile && row < p.m, ec, er[ps]);
+        epi_apply<EPI, XG>(p, row, grp, c0, v[ps], cols && r < rows_in_tile && row < p.m, ec, er[ps]);
     }
     if (EPI & EPI_SCORE) {
         // Every tile's partials are stored (device-coherent) before its arrival counts; the last

@@ -143,6 +143,9 @@ int wide_height(int m, int n, int cus);
 bool gemm_group_takes(int bm, int k);
 int gemm_group_height(int m, int n, int k, int cus);
 void gemm_group_launch(const GemmParams& p, int epi, int bm, hipStream_t stream);
+// The same on tiles of 16 rows x 32 columns.
+bool gemm_group0_takes(int m, int n, int k, int cus, int epi);
+void gemm_group0_launch(const GemmParams& p, int epi, hipStream_t stream);
 // The same on tiles of 128 columns.
 int gemm_group2_height(int m, int n, int k, int cus, int epi);
 void gemm_group2_launch(const GemmParams& p, int epi, int bm, hipStream_t stream);

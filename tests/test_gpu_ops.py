@@ -200,7 +200,11 @@ GROUP = [("lnrope", 559, 2304, 768), ("lngeglu", 560, 2304, 576), ("lnbias", 561
          # two column groups: 64 rows (three lines), 48 and 64 (four and five), 32 and 48 (six)
          ("lnrope", 673, 2304, 768), ("lngeglu", 895, 2304, 576), ("biasresstats", 2688, 768, 704),
          ("lnbias", 449, 2304, 832), ("lnbiasrelu", 2625, 768, 1024), ("resstats", 1345, 768, 1152),
-         ("biasresstats", 2687, 768, 1280), ("resstats", 1009, 768, 1536), ("resstats", 2015, 768, 1344)]
+         ("biasresstats", 2687, 768, 1280), ("resstats", 1009, 768, 1536), ("resstats", 2015, 768, 1344),
+         # half a column group, 16 rows: one row, a row past a tile, the most rows that fit and one more
+         ("lnbiasgelu", 6, 768, 768), ("rope", 1, 192, 256), ("lnrope", 17, 192, 320), ("lngeglu", 48, 2304, 1152),
+         ("lngeglu", 49, 2304, 768), ("lnbiasrelu", 80, 1536, 1024), ("lnbias", 335, 384, 384),
+         ("lnrope", 47, 2304, 1536)]
 
 
 @pytest.mark.parametrize("kind,m,n,k", GROUP, ids=["-".join(map(str, g)) for g in GROUP])
