@@ -87,6 +87,8 @@ __device__ __forceinline__ void gemm_group_tile(const GemmParams& p, int task, c
         }
     }
 
+    __builtin_amdgcn_sched_barrier(0);  // (the wait below counts w's loads as issued after the copies)
+
     // The epilogue's other inputs, in flight with the operands.
     const int c0 = (tid & 7) * 4;
     EpiCol ec;

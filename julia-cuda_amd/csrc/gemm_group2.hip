@@ -23,7 +23,8 @@ int gemm_group2_height(int m, int n, int k, int cus, int epi) {
 
 // Tiles of 16 rows x 32 columns where that grid is at most a block a CU: a CU then takes in half of
 // w's 64 columns (MI355X, us, 16 x 64 tiles / this: the scorer's lin1 on 6 rows 4.1 / 3.6, linear1 on 80
-// rows 3.9 / 3.5, qkv on 48 rows 3.95 / 3.4, at d = 384 on 100 rows 4.0 / 3.2). Not with output statistics (a group's are one block's) or the score.
+// rows 3.9 / 3.5, qkv on 48 rows 3.95 / 3.4, at d = 384 on 100 rows 4.0 / 3.2). Not with output
+// statistics (a group's are one block's) or the score.
 bool gemm_group0_takes(int m, int n, int k, int cus, int epi) {
     return k >= 256 && group_rows_max(group_lines(k)) && !(epi & (EPI_STATS | EPI_SCORE | EPI_GATHER)) &&
            (long)(n / 32) * (((long)m + 15) / 16) <= cus;
