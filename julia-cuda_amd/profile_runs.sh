@@ -2,15 +2,16 @@
 # The profiler runs behind profiles/ (per-step kernels only: no cooperative launch runs under
 # rocprofv3). Usage, from the repository root on the GPU box:
 #     bash julia-cuda_amd/profile_runs.sh OUT [parts]
-# parts (default all): trace (bench.py's timed runs under --kernel-trace: the rocprofv3 duration
+# parts (default: both): trace (bench.py's timed runs under --kernel-trace: the rocprofv3 duration
 # of every HIP-event figure in the bench line), traffic (FETCH_SIZE / WRITE_SIZE passes of the
-# 293-token roofline kernels, calibrated by the library's copy kernel), forward (kernel
-# statistics of the 293-token forward pass, per-step path). Writes raw output under OUT and the
+# 293-token roofline kernels, calibrated by the library's copy kernel). The
+# graph-replayed forward pass is not profiled: a run of it under rocprofv3 ended in a host
+# segmentation fault inside a HIP call, its cause not known. Writes raw output under OUT and the
 # summaries bench.py reads under OUT/profiles_new (copy them to profiles/).
 set -o pipefail
 R=$(cd "$(dirname "$0")/.." && pwd)
 OUT=$(cd "$1" && pwd) || exit 2
-PARTS=${2:-trace,traffic,forward}
+PARTS=${2:-trace,traffic}
 NEW=$OUT/profiles_new
 mkdir -p $NEW
 cd /tmp && export TMPDIR=/tmp
@@ -34,8 +35,7 @@ if has traffic; then
     done
 fi
 if has forward; then
-    echo "profile: the 293-token forward pass, per-step kernels" >&2
-    timeout -k 10 300 rocprofv3 --kernel-trace --stats -f csv -d $OUT/fwd -o fwd -- \
-        python3 $R/bench.py --quick --path per-step --steps 200 --warmup 20 > $OUT/fwd.log 2>&1 || exit $?
+    echo "profile: the graph-replayed forward pass is not run under the profiler (see above)" >&2
+    exit 2
 fi
 echo "profile: done" >&2
