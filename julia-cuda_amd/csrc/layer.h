@@ -138,9 +138,11 @@ public:
     // 64-query tile, run by the kernel's large-batch instance (two blocks a CU).
     static bool is_big(const LayerPlan& plan, int m);
     static int big_mode(const LayerPlan& plan, int m);  // the kernel instance (layer.hip)
+    // The rows of the wide tiles (bm 256 in a plan) a launch on m rows takes: 192 or 224.
+    int wide_rows(int m, int d, int inter) const;
 
 private:
-    int cus_ = 0, per_cu_ = 0, per_cu_big_ = 0, per_cu_big256_ = 0, lds_max_ = 0;
+    int cus_ = 0, per_cu_ = 0, per_cu_big_ = 0, per_cu_wide_ = 0, lds_max_ = 0;
     bool lat48_ok_ = false;  // the 48-row instance fits as many blocks a CU as the plain one
     uint32_t* bar_ = nullptr;  // BAR_WORDS words
     // Launch through hipLaunchCooperativeKernel (true), or as a plain launch of the same

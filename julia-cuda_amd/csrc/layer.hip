@@ -145,6 +145,9 @@ __device__ __forceinline__ jh_half* x_out_of(const EncParams& P, int l) {
     return P.xa + (size_t)(2 * l + 1) * P.x_stride;
 }
 
+// The columns of a tile of `rows` rows: a latency tile, the 128 x 128 or a wide tile.
+__host__ __device__ constexpr int tile_cols(int rows) { return rows < 128 ? 64 : rows == 128 ? 128 : WIDE_BN; }
+
 __device__ __forceinline__ GemmParams make_gemm(const EncParams& P, int g, const LayerDesc& L,
                                                 int l) {
     GemmParams p{};
@@ -165,7 +168,7 @@ __device__ __forceinline__ GemmParams make_gemm(const EncParams& P, int g, const
         p.a = P.mid, p.w = L.wo_mlp, p.c = x_out_of(P, l), p.res = x_attn_of(P, l);
         p.n = P.d, p.k = P.inter, p.stats_out = P.stats_mlp;
     }
-    p.tiles_n = p.n / (P.bm[g] >= 128 ? P.bm[g] : 64);
+    p.tiles_n = p.n / tile_cols(P.bm[g]);
     p.tiles_m = (P.m + P.bm[g] - 1) / P.bm[g];
     return p;
 }
@@ -196,7 +199,7 @@ __device__ __forceinline__ GemmParams make_head_gemm(const EncParams& P, int g, 
         p.a = hx(2 * M.head_layers), p.w = M.lin1, p.c = M.hs, p.n = P.d, p.k = P.d;
         p.stats_in = P.stats_attn, p.colsum = M.lin1_colsum, p.bias = M.lin1_b;
     }
-    p.tiles_n = p.n / (P.hbm[g] >= 128 ? P.hbm[g] : 64);
+    p.tiles_n = p.n / tile_cols(P.hbm[g]);
     p.tiles_m = (P.m + P.hbm[g] - 1) / P.hbm[g];
     return p;
 }
@@ -206,10 +209,18 @@ __device__ __forceinline__ int gemm_tasks(const GemmParams& g) {
 }
 
 // The kernel's instances: MODE_LAT takes every plan (256 threads, one block a CU); MODE_BIG128
-// and MODE_BIG256 the large-batch plans of 128 x 128 tiles (256 threads, two blocks a CU) and of
-// 256 x 256 tiles (512 threads, one block a CU), with only the throughput tiles and the streaming
+// and MODE_WIDE the large-batch plans of 128 x 128 tiles (256 threads, two blocks a CU) and of
+// the wide tiles (512 threads, one block a CU), with only the throughput tiles and the streaming
 // attention tile compiled in.
-constexpr int MODE_LAT = 0, MODE_BIG128 = 1, MODE_BIG256 = 2;
+//
+// MODE_WIDE's tiles are WROWS = 192 or 224 rows high (LayerKernel::wide_rows picks by the rounds of
+// tiles), one height for all GEMMs of a launch, named 256 in the plans. 256-row tiles hold 64
+// accumulators and as many operand registers a lane: with nine phases inlined into one kernel 101
+// registers were spilled (192 rows: 4, 224: 40), some of them in the attention loop, and a batch
+// of a round or two of tiles has fewer of them. Measured (MI355X, a batched pass through the
+// whole model, us, 256 rows / 192 / 224): 2076 rows 3195 / 2660 / 2958, 3778 3632 / 3010 / 3355,
+// 5774 3995 / 4052 / 3766, 9291 5617 / 4622 / 5140, 18530 8470 / 8455 / 7771.
+constexpr int MODE_LAT = 0, MODE_BIG128 = 1, MODE_WIDE = 2;
 // MODE_LAT48: MODE_LAT with the 48-row latency tile compiled in for qkv and wi, for the plans
 // that take it (an instance of its own: the code it adds shifts the register and spill layout
 // of the whole kernel, which the other plans measured slower with).
@@ -220,13 +231,13 @@ constexpr int MODE_LAT48 = 3;
 template <int EPI, int MODE>
 constexpr bool T48 = MODE == MODE_LAT48 && (EPI == EPI_K_ROPE || EPI == EPI_K_LNROPE || EPI == EPI_K_LNGEGLU);
 
-// bm 16/32/48/64: the latency tile with its weights in LDS; 128 and 256: the throughput tiles
+// bm 16/32/48/64: the latency tile with its weights in LDS; 128 and H: the throughput tiles
 // (large batches), which stage both operands themselves.
-template <int EPI, bool AX, int MODE>
+template <int EPI, bool AX, int MODE, int WROWS>
 __device__ __forceinline__ void gemm_phase(const GemmParams& g, int bm, char* lds, bool pre,
                                            uint32_t* s_last, uint64_t* sub) {
-    if (MODE == MODE_BIG256) {
-        gemm_wide_run<256, EPI, AX, true>(g, blockIdx.x, gridDim.x, lds, sub);
+    if constexpr (MODE == MODE_WIDE) {
+        gemm_wide_run<WROWS, EPI, AX, true>(g, blockIdx.x, gridDim.x, lds, sub);
         return;
     }
     const int T = gemm_tasks(g);
@@ -247,10 +258,10 @@ __device__ __forceinline__ void gemm_phase(const GemmParams& g, int bm, char* ld
     }
 }
 
-template <int MODE>
-__global__ __launch_bounds__(MODE == MODE_BIG256 ? 512 : 256, MODE == MODE_BIG128 ? 2 : 1)
+template <int MODE, int WROWS = 0>
+__global__ __launch_bounds__(MODE == MODE_WIDE ? 512 : 256, MODE == MODE_BIG128 ? 2 : 1)
 void encoder_kernel(EncParams P) {
-    constexpr bool BIG = MODE == MODE_BIG128 || MODE == MODE_BIG256;
+    constexpr bool BIG = MODE == MODE_BIG128 || MODE == MODE_WIDE;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     uint32_t* s_last = (uint32_t*)(lds + P.lds_main);
     uint32_t g0 = 0, nb = 0;
@@ -282,7 +293,7 @@ void encoder_kernel(EncParams P) {
             for (int t = blockIdx.x; t < T; t += gridDim.x)
                 attention_slice_tile<false, true>(at, t, lds, gkeys, t == (int)blockIdx.x ? su0 : nullptr);
         } else if (BIG || at.chunks == 1) {  // (the large-batch instances have one key range)
-            constexpr int NW = MODE == MODE_BIG256 ? 8 : 4;
+            constexpr int NW = MODE == MODE_WIDE ? 8 : 4;
             const int T = ((P.m + 16 * NW - 1) / (16 * NW)) * heads;
             for (int t = blockIdx.x; t < T; t += gridDim.x)
                 attention_stream_tile<true, NW>(at, t, lds);
@@ -318,9 +329,9 @@ void encoder_kernel(EncParams P) {
         if (on(0)) {
             stamp(prof, 0);
             if (gq.colsum)
-                gemm_phase<EPI_K_LNROPE, false, MODE>(gq, P.bm[0], lds, pre, s_last, sub(0));
+                gemm_phase<EPI_K_LNROPE, false, MODE, WROWS>(gq, P.bm[0], lds, pre, s_last, sub(0));
             else
-                gemm_phase<EPI_K_ROPE, false, MODE>(gq, P.bm[0], lds, pre, s_last, sub(0));
+                gemm_phase<EPI_K_ROPE, false, MODE, WROWS>(gq, P.bm[0], lds, pre, s_last, sub(0));
             pre = false;
             stamp_end(prof, 0);
             if (on(1)) sync(nothing);
@@ -339,7 +350,7 @@ void encoder_kernel(EncParams P) {
         }
         if (on(2)) {
             stamp(prof, 4);
-            gemm_phase<EPI_K_RESSTATS, false, MODE>(go, P.bm[1], lds, pre, s_last, sub(1));
+            gemm_phase<EPI_K_RESSTATS, false, MODE, WROWS>(go, P.bm[1], lds, pre, s_last, sub(1));
             pre = false;
             stamp_end(prof, 2);
             if (on(3)) {
@@ -349,7 +360,7 @@ void encoder_kernel(EncParams P) {
         }
         if (on(3)) {
             stamp(prof, 6);
-            gemm_phase<EPI_K_LNGEGLU, false, MODE>(gi, P.bm[2], lds, pre, s_last, sub(2));
+            gemm_phase<EPI_K_LNGEGLU, false, MODE, WROWS>(gi, P.bm[2], lds, pre, s_last, sub(2));
             pre = false;
             stamp_end(prof, 3);
             if (on(4)) {
@@ -359,7 +370,7 @@ void encoder_kernel(EncParams P) {
         }
         if (on(4)) {
             stamp(prof, 8);
-            gemm_phase<EPI_K_RESSTATS, true, MODE>(gm, P.bm[3], lds, pre, s_last, sub(3));
+            gemm_phase<EPI_K_RESSTATS, true, MODE, WROWS>(gm, P.bm[3], lds, pre, s_last, sub(3));
             pre = false;
             stamp_end(prof, 4);
         }
@@ -387,25 +398,25 @@ void encoder_kernel(EncParams P) {
                          g1 = make_head_gemm(P, 2, H, h), g2 = make_head_gemm(P, 3, H, h);
         pre = prefetch(gi, P.hbm[0]);
         if (pre) sync(fetch_first(gi)); else sync(nothing);
-        gemm_phase<EPI_K_LNBIAS, false, MODE>(gi, P.hbm[0], lds, pre, s_last, nullptr);
+        gemm_phase<EPI_K_LNBIAS, false, MODE, WROWS>(gi, P.hbm[0], lds, pre, s_last, nullptr);
         sync(nothing);
         attend(AttnParams{M.hqa + (size_t)h * P.q_stride, M.hoa + (size_t)h * P.o_stride, P.m, P.d,
                           0, P.kv[0], P.ws, P.counters, P.seg},
                nullptr);
         pre = prefetch(go, P.hbm[1]);
         if (pre) sync(fetch_first(go)); else sync(nothing);
-        gemm_phase<EPI_K_BIASRESSTATS, false, MODE>(go, P.hbm[1], lds, pre, s_last, nullptr);
+        gemm_phase<EPI_K_BIASRESSTATS, false, MODE, WROWS>(go, P.hbm[1], lds, pre, s_last, nullptr);
         pre = prefetch(g1, P.hbm[2]);
         if (pre) sync(fetch_first(g1)); else sync(nothing);
-        gemm_phase<EPI_K_LNBIASRELU, false, MODE>(g1, P.hbm[2], lds, pre, s_last, nullptr);
+        gemm_phase<EPI_K_LNBIASRELU, false, MODE, WROWS>(g1, P.hbm[2], lds, pre, s_last, nullptr);
         pre = prefetch(g2, P.hbm[3]);
         if (pre) sync(fetch_first(g2)); else sync(nothing);
-        gemm_phase<EPI_K_BIASRESSTATS, true, MODE>(g2, P.hbm[3], lds, pre, s_last, nullptr);
+        gemm_phase<EPI_K_BIASRESSTATS, true, MODE, WROWS>(g2, P.hbm[3], lds, pre, s_last, nullptr);
     }
     const GemmParams gs = make_head_gemm(P, 4, HeadDesc{}, 0);
     pre = prefetch(gs, P.hbm[4]);
     if (pre) sync(fetch_first(gs)); else sync(nothing);
-    gemm_phase<EPI_K_LNBIASGELU, false, MODE>(gs, P.hbm[4], lds, pre, s_last, nullptr);
+    gemm_phase<EPI_K_LNBIASGELU, false, MODE, WROWS>(gs, P.hbm[4], lds, pre, s_last, nullptr);
     sync(nothing);
     for (int i = blockIdx.x * nwv + wv; i < M.n_markers; i += gridDim.x * nwv)
         score_row<4>((const f16*)M.hs, P.m, P.d, (const f16*)M.lin2, M.lin2_b, M.markers, i,
@@ -446,7 +457,7 @@ int LayerKernel::lds_bytes(const LayerPlan& plan, int d, int inter, int m, int w
 
 // The large-batch instances' LDS: the throughput tile or the streaming attention tile.
 static int big_lds_bytes(int bm) {
-    const int g = bm == 256 ? Wide<256>::LDS_BYTES : Big::LDS_BYTES;
+    const int g = bm == 256 ? std::max<int>(Wide<224>::LDS_BYTES, Wide<192>::LDS_BYTES) : Big::LDS_BYTES;
     return (std::max<int>(g, ATT_STREAM_LDS) + 15) / 16 * 16;
 }
 
@@ -457,7 +468,7 @@ void LayerKernel::init(int cus, int lds_max) {
     const char* skew = getenv("JULIA_HIP_TEST_BARRIER_SKEW");
     skew_ = skew && strcmp(skew, "1") == 0 ? 1u : 0u;
     lds_max_ = lds_max - 16;  // the split-K flag after the main area
-    per_cu_ = per_cu_big_ = per_cu_big256_ = 0;
+    per_cu_ = per_cu_big_ = per_cu_wide_ = 0;
     auto occupancy = [](const void* k, int threads, int lds) {
         if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) {
             (void)hipGetLastError();
@@ -473,8 +484,9 @@ void LayerKernel::init(int cus, int lds_max) {
                 occupancy(reinterpret_cast<const void*>(encoder_kernel<MODE_LAT48>), 256, lds_max) >= per_cu_;
     per_cu_big_ = occupancy(reinterpret_cast<const void*>(encoder_kernel<MODE_BIG128>), 256,
                             big_lds_bytes(128) + 16);
-    per_cu_big256_ = occupancy(reinterpret_cast<const void*>(encoder_kernel<MODE_BIG256>), 512,
-                               big_lds_bytes(256) + 16);
+    per_cu_wide_ = occupancy(reinterpret_cast<const void*>(encoder_kernel<MODE_WIDE, 192>), 512, big_lds_bytes(256) + 16);
+    per_cu_wide_ = std::min(per_cu_wide_, occupancy(reinterpret_cast<const void*>(encoder_kernel<MODE_WIDE, 224>), 512,
+                                                    big_lds_bytes(256) + 16));
 }
 
 // Per GEMM the tile height and split-K with the least modelled time on a grid of one block per
@@ -524,7 +536,7 @@ static bool head_plan(const LayerPlan& plan, int m, int d, int ff, int cus, int 
     const int mode = LayerKernel::big_mode(plan, m);
     for (int g = 0; g < 5; g++) {
         if (mode != MODE_LAT) {
-            const int t = mode == MODE_BIG256 ? 256 : 128;
+            const int t = mode == MODE_WIDE ? 256 : 128;
             if (cols[g] % t || ks[g] % 64 || (ln[g] && ks[g] > GEMM_BIG_LN_MAX_K)) return false;
             bm[g] = t, splits[g] = 1;
         } else {
@@ -546,7 +558,7 @@ LayerPlan LayerKernel::default_plan(int m, int d, int inter) const {
     shapes(d, inter, cols, ks);
     for (int g = 0; g < 4; g++) {
         // Large batches: the throughput tile (LayerNorm epilogues, qkv and wi, need K <= 1024),
-        // 256 x 256 where every GEMM's columns allow it (big_tiles below), else 128 x 128.
+        // the wide tiles where every GEMM's columns allow it (below), else 128 x 128.
         const bool ln = g == 0 || g == 2;
         if (m > ATT_SLICE_ROWS && cols[g] % 128 == 0 && ks[g] % 64 == 0 &&
             (!ln || ks[g] <= GEMM_BIG_LN_MAX_K) && Big::LDS_BYTES <= lds_max_) {
@@ -557,12 +569,26 @@ LayerPlan LayerKernel::default_plan(int m, int d, int inter) const {
     }
     p.kv[0] = attention_chunks(m, d, 0, cus_);
     p.kv[1] = 1;
-    // All four on 256 x 256 tiles (one 512-thread block a CU) when they all take them.
-    bool all256 = per_cu_big256_ > 0 && big_lds_bytes(256) <= lds_max_;
+    // All four on wide tiles (one 512-thread block a CU) when they all take them.
+    bool all256 = per_cu_wide_ > 0 && big_lds_bytes(256) <= lds_max_;
     for (int g = 0; g < 4; g++) all256 = all256 && p.bm[g] == 128 && cols[g] % 256 == 0;
     if (all256)
         for (int g = 0; g < 4; g++) p.bm[g] = 256;
     return p;
+}
+
+// The height of the wide tiles of a launch on m rows: the one whose rounds over the CUs take
+// less, a tile's time growing as its rows plus about 53 (wide_height in gemm_wide.hip) and its K.
+int LayerKernel::wide_rows(int m, int d, int inter) const {
+    int cols[4], ks[4];
+    shapes(d, inter, cols, ks);
+    auto cost = [&](int h) {
+        long c = 0;
+        for (int g = 0; g < 4; g++)
+            c += ((long)(cols[g] / WIDE_BN) * ((m + h - 1) / h) + cus_ - 1) / cus_ * (h + 53) * ks[g];
+        return c;
+    };
+    return cost(224) < cost(192) ? 224 : 192;
 }
 
 size_t LayerKernel::ws_floats(int max_m, int d, int inter, int head_ff) const {
@@ -602,13 +628,14 @@ int LayerKernel::grid(const LayerArgs& a, const LayerPlan& plan) const {
     shapes(a.d, a.inter, cols, ks);
     long most = (long)((a.m + 15) / 16) * (a.d / 64);  // attention slices
     most = std::max(most, (long)((a.m + 63) / 64) * (a.d / 64) * std::max(plan.kv[0], plan.kv[1]));
-    for (int g = 0; g < 4; g++)
-        most = std::max(most, (long)(cols[g] / (plan.bm[g] >= 128 ? plan.bm[g] : 64)) *
-                                  ((a.m + plan.bm[g] - 1) / plan.bm[g]) * plan.splits[g]);
+    const int mode = big_mode(plan, a.m);
+    for (int g = 0; g < 4; g++) {
+        const int rows = mode == MODE_WIDE ? wide_rows(a.m, a.d, a.inter) : plan.bm[g];
+        most = std::max(most, (long)(cols[g] / tile_cols(rows)) * ((a.m + rows - 1) / rows) * plan.splits[g]);
+    }
     // Enough blocks for the largest phase's tasks in one round if they fit (a multiple of 8, so
     // that the task-to-XCD map is even), else every resident block.
-    const int mode = big_mode(plan, a.m);
-    const int per_cu = mode == MODE_BIG256 ? per_cu_big256_ : mode == MODE_BIG128 ? per_cu_big_ : per_cu_;
+    const int per_cu = mode == MODE_WIDE ? per_cu_wide_ : mode == MODE_BIG128 ? per_cu_big_ : per_cu_;
     const long grid = std::min<long>((long)per_cu * cus_, (most + 7) / 8 * 8);
     return (int)std::max<long>(grid, 1);
 }
@@ -636,12 +663,12 @@ bool LayerKernel::launch(const LayerArgs& a, const LayerPlan& plan, const Scratc
     const int mode = big_mode(plan, a.m);
     bool any256 = false;
     for (int g = 0; g < 4; g++) any256 = any256 || plan.bm[g] == 256;
-    if (any256 && mode != MODE_BIG256)
-        fail("256 x 256 tiles take every GEMM, more than " + std::to_string(ATT_SLICE_ROWS) +
+    if (any256 && mode != MODE_WIDE)
+        fail("the wide tiles take every GEMM, more than " + std::to_string(ATT_SLICE_ROWS) +
              " rows and one key range: " + plan.str());
-    if ((mode == MODE_BIG128 && per_cu_big_ <= 0) || (mode == MODE_BIG256 && per_cu_big256_ <= 0))
+    if ((mode == MODE_BIG128 && per_cu_big_ <= 0) || (mode == MODE_WIDE && per_cu_wide_ <= 0))
         fail("the encoder kernel's large-batch instance does not fit on a CU");
-    int lds = mode == MODE_BIG256   ? big_lds_bytes(256)
+    int lds = mode == MODE_WIDE   ? big_lds_bytes(256)
                     : mode == MODE_BIG128 ? big_lds_bytes(128)
                                           : lds_bytes(plan, a.d, a.inter, a.m, window);
     if (lds > lds_max_) fail("the plan's weight tiles do not fit the LDS: " + plan.str());
@@ -740,7 +767,8 @@ bool LayerKernel::launch(const LayerArgs& a, const LayerPlan& plan, const Scratc
     P.stats_attn = a.stats_attn, P.stats_mlp = a.stats_mlp;
     P.pos = a.pos, P.seg = a.seg;
     P.m = a.m, P.d = a.d, P.inter = a.inter, P.rope_rows = a.rope_rows, P.eps = a.eps;
-    for (int g = 0; g < 4; g++) P.bm[g] = plan.bm[g], P.splits[g] = plan.splits[g];
+    const int rows = mode == MODE_WIDE ? wide_rows(a.m, a.d, a.inter) : 0;  // every GEMM's, with the wide tiles
+    for (int g = 0; g < 4; g++) P.bm[g] = rows ? rows : plan.bm[g], P.splits[g] = plan.splits[g];
     P.kv[0] = plan.kv[0], P.kv[1] = plan.kv[1];
     P.ws = s.ws, P.counters = s.counters;
     P.phases = phases;
@@ -750,7 +778,7 @@ bool LayerKernel::launch(const LayerArgs& a, const LayerPlan& plan, const Scratc
     P.barriers = barriers * a.count + (a.count - 1);
     if (M) {  // after embed, after the last layer, five a head layer, before lin1 and the score
         P.model = 1, P.M = *M;
-        for (int g = 0; g < 5; g++) P.hbm[g] = hbm[g], P.hsplits[g] = hsplits[g];
+        for (int g = 0; g < 5; g++) P.hbm[g] = rows ? rows : hbm[g], P.hsplits[g] = hsplits[g];
         P.barriers += 4 + 5 * M->head_layers;
         lds = lds_model;
     }
@@ -764,11 +792,12 @@ bool LayerKernel::launch(const LayerArgs& a, const LayerPlan& plan, const Scratc
     const int grid_blocks = grid(a, plan);
     const bool uses48 = mode == MODE_LAT && (plan.bm[0] == 48 || plan.bm[2] == 48);
     void* args[] = {&P};
-    const void* kernel = mode == MODE_BIG256   ? reinterpret_cast<const void*>(encoder_kernel<MODE_BIG256>)
+    const void* kernel = rows == 224 ? reinterpret_cast<const void*>(encoder_kernel<MODE_WIDE, 224>)
+                         : rows ? reinterpret_cast<const void*>(encoder_kernel<MODE_WIDE, 192>)
                          : mode == MODE_BIG128 ? reinterpret_cast<const void*>(encoder_kernel<MODE_BIG128>)
                          : uses48 ? reinterpret_cast<const void*>(encoder_kernel<MODE_LAT48>)
                                                : reinterpret_cast<const void*>(encoder_kernel<MODE_LAT>);
-    const dim3 threads(mode == MODE_BIG256 ? 512 : 256);
+    const dim3 threads(mode == MODE_WIDE ? 512 : 256);
     hipError_t e;
     if (coop_) {
         e = hipLaunchCooperativeKernel(kernel, dim3(grid_blocks), threads, args, lds + 16, stream);
@@ -798,7 +827,7 @@ int LayerKernel::big_mode(const LayerPlan& plan, int m) {
     if (m <= ATT_SLICE_ROWS || plan.kv[0] != 1 || plan.kv[1] != 1) return MODE_LAT;
     for (int g = 1; g < 4; g++)
         if (plan.bm[g] != plan.bm[0]) return MODE_LAT;
-    return plan.bm[0] == 256 ? MODE_BIG256 : plan.bm[0] == 128 ? MODE_BIG128 : MODE_LAT;
+    return plan.bm[0] == 256 ? MODE_WIDE : plan.bm[0] == 128 ? MODE_BIG128 : MODE_LAT;
 }
 
 bool LayerKernel::barrier_timed_out() {

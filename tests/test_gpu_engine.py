@@ -271,6 +271,32 @@ def test_batched_encoder_on_256_tiles(torch_cuda):
     e.close()
 
 
+@pytest.mark.parametrize("rows", [5376, 5377])
+def test_persistent_kernel_on_either_wide_height(torch_cuda, rows):
+    """The persistent kernel's wide instances on either side of the row count where their height
+    changes on 256 CUs (28 tiles of 192 rows x 9 column tiles are the last single round; a row more
+    takes 224-row tiles, one of them of a single row): the encoder against the per-step
+    kernels, the whole model's logits against the per-step pass's."""
+    c = dict(d=768, layers=2, inter=1152, vocab=1000, head_ff=1536, max_positions=4096, seed=19)
+    e = jh.Engine(spec(c), max_length=1024, batch_rows=rows)
+    rng = np.random.default_rng(rows)
+    lens = [1024, 513, 700, 1, 900, 1024, 17, 640]
+    lens.append(rows - sum(lens))
+    reqs = [(rng.integers(0, c["vocab"], n).astype(np.uint32), rng.integers(0, n, 4).astype(np.uint32), i % 3)
+            for i, n in enumerate(lens)]
+    seqs = [r[0] for r in reqs]
+    xs, _ = e.encode_batch(seqs, layer_fused=False)
+    xf, ms = e.encode_batch(seqs, layer_fused=True)
+    say(f"wide layer kernel: {rows} rows, {ms:.3f} GPU ms")
+    compare(f32(xf), f32(xs), 1e-2, 5e-2, what=f"layer kernel vs per-step, {rows} rows")
+    assert e.model_kernel(rows)
+    lf, _ = e.run(reqs, layer_fused=True, batched=True)
+    ls, _ = e.run(reqs, batched=True)
+    a, b = np.concatenate(lf), np.concatenate(ls)
+    assert np.isfinite(a).all() and np.abs(a - b).max() <= 1e-2
+    e.close()
+
+
 def test_whole_model_on_256_tiles(torch_cuda):
     """The whole-model launch on the 256 x 256 instance (config 4's widths, head_ff 1536, a
     batched pass past 2048 rows): every head GEMM on the throughput tile, attention bounded to

@@ -6,6 +6,9 @@ the reference's own known-answer tests; the C ABI's error paths that need no GPU
 import ctypes
 import os
 import re
+import struct
+import subprocess
+import tempfile
 
 import numpy as np
 import pytest
@@ -24,6 +27,37 @@ def test_library_exports_every_declared_symbol():
     L = jh.lib()
     for name in declared:
         assert getattr(L, name) is not None
+
+
+def kernel_spills():
+    """{kernel: vector registers spilled} from the metadata of the code objects in the library."""
+    tool = "/opt/rocm/llvm/bin/llvm-readelf"
+    if not os.path.exists(tool):
+        pytest.skip("no llvm-readelf")
+    data, out = open(jh.LIB_PATH, "rb").read(), {}
+    at = data.find(b"\x7fELF", 1)
+    while at >= 0:
+        if struct.unpack_from("<H", data, at + 18)[0] == 224:  # EM_AMDGPU
+            shoff, shentsize, shnum = (struct.unpack_from(f, data, at + o)[0] for f, o in (("<Q", 40), ("<H", 58), ("<H", 60)))
+            with tempfile.NamedTemporaryFile() as f:
+                f.write(data[at:at + shoff + shentsize * shnum])
+                f.flush()
+                notes = subprocess.run([tool, "--notes", f.name], capture_output=True, text=True, check=True).stdout
+            for k in notes.split("- .agpr_count")[1:]:
+                name = re.search(r"\n    \.name:\s+(\S+)", k).group(1)
+                out[name] = int(re.search(r"\.vgpr_spill_count:\s+(\d+)", k).group(1))
+        at = data.find(b"\x7fELF", at + 4)
+    return out
+
+
+def test_the_encoder_kernel_keeps_its_registers():
+    """Every phase of the persistent kernel is inlined into each of its instances, so a tile that
+    takes the last registers by itself spills there, in the phases' loops too: 256-row wide tiles
+    spilled 101 (and cost 2 to 15% of a batched pass), the heights it has 1 and 40, none of them
+    in a loop of MFMAs over K."""
+    spills = {k: v for k, v in kernel_spills().items() if "encoder_kernel" in k}
+    assert len(spills) == 5, spills
+    assert max(spills.values()) <= 48, spills
 
 
 def test_tier():
