@@ -205,34 +205,6 @@ def path_ms(t):
     return {"mean": round(t[0], 4), "median": round(t[1], 4), "wall": round(t[2], 4)}
 
 
-def gemm_instance(m, n, k, bm, epi, cus):
-    """The kernel instance the engine launches for an m x n x k GEMM with tile height bm (one
-    K split)."""
-    ks, ceil = k / 768, lambda a, b: -(-a // b)
-    lines = max(2, ceil(k // 64, 4))  # the grouped latency kernel's instance and its highest tile
-    top = {2: 128, 3: 96, 4: 64, 5: 64, 6: 48}.get(lines, 0) if k >= 256 else 0
-    if top and not ("stats" in epi or "score" in epi) and n // 32 * ceil(m, 16) <= cus:
-        return f"gemm_group<16, {jh.EPI[epi]}, {lines}, 0>"
-    for h in (16, 32, 48, 64, 80, 96, 128):
-        if h <= top and n // 64 * ceil(m, h) <= cus:
-            return f"gemm_group<{h}, {jh.EPI[epi]}, {lines}, 1>"
-    low = {3: 64, 4: 48, 5: 48, 6: 32}.get(lines, 256)
-    for h in (32, 48, 64):
-        if n % 128 == 0 and low <= h <= top and not ("ln" in epi and k > 1024) and n // 128 * ceil(m, h) <= cus:
-            return f"gemm_group<{h}, {jh.EPI[epi]}, {lines}, 2>"
-    if bm >= 128:  # the throughput kernel the launch takes (gemm_pick in csrc/gemm.hip)
-        l128 = ceil(n // 128 * ceil(m, 128), cus)
-        c128 = 2 + 8.5 * ks if l128 == 1 else 2.5 + 7.6 * ks * l128
-        rounds = lambda h: ceil(n // 256 * ceil(m, h), cus)
-        h = min((256, 224, 192, 160), key=lambda h: rounds(h) * (h + 53))
-        if n % 256 == 0 and 4.5 + rounds(h) * (0.2 + h / 80 + ks * (3.2 + h / 20)) < c128:
-            return f"gemm_wide<{h}, {jh.EPI[epi]}, false>"
-        return f"gemm_big<{jh.EPI[epi]}, false>"
-    if (n // 64) * -(-m // bm) <= cus and k >= 256:  # the eight-wave instance: a block a CU at most
-        return f"gemm_lat1<{bm}, {jh.EPI[epi]}>"
-    return f"gemm_lat<{bm}, {jh.EPI[epi]}>"
-
-
 def roofline(kern, steps, kname):
     """The roofline entry of one kernel instance at 293 tokens over the steps that run it: the
     algorithmic bytes (or flops) of the forward's launches of it over their HIP-event time
@@ -366,8 +338,7 @@ def main():
     if "kernels" in sections:
         kern = {}
         for step, (n, k, epi, cnt) in STEP_SHAPES.items():
-            cfg = list(jh.gemm_choose(293, n, k, info.cus, epi))
-            kname = gemm_instance(293, n, k, cfg[0], epi, info.cus)
+            *cfg, kname = jh.gemm_pick(293, n, k, info.cus, epi)
             mn, md = time_step(eng, step, 293, f"{step}@293", kname)
             kern[step] = dict(us=round(md, 3), us_min=round(mn, 3), per_forward=cnt, kernel=kname,
                               bytes=gemm_bytes(293, n, k, epi), flops=2 * 293 * n * k, config=cfg)
@@ -432,7 +403,7 @@ def main():
                         grid[f"{bm}/{sp}"] = None
             _, md = jh.time_gemm(gargs, scratch=scr, warmup=5, batches=5, per_batch=20)
             c2[step] = {"epilogue": epi, "us_by_bm_split": grid,
-                        "chosen": list(jh.gemm_choose(M2, n, k, info.cus, epi)),
+                        "chosen": jh.gemm_pick(M2, n, k, info.cus, epi)[2],
                         "chosen_us": round(md, 2),
                         "TFLOPs": round(2 * M2 * n * k / (md * 1e-6) / 1e12, 1)}
             for b in (a, w, c, st_in, cs, st_out):
@@ -465,8 +436,7 @@ def main():
         eng_big = jh.Engine(BIG_SPEC, max_length=18752)
         for m in (4096, 8192, 18752):
             for step, (n, k, epi, _) in STEP_SHAPES.items():
-                cfg = list(jh.gemm_choose(m, n, k, info.cus, epi))
-                kname = gemm_instance(m, n, k, cfg[0], epi, info.cus)
+                *cfg, kname = jh.gemm_pick(m, n, k, info.cus, epi)
                 mn, md = time_step(eng_big, step, m, f"{step}@{m}", kname, warmup=5, batches=5,
                                    per_batch=8)
                 fl = 2 * m * n * k

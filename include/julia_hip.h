@@ -131,8 +131,8 @@ typedef struct {
 
 /* src/gemm.rs:126-137 `Config`: tile height (16, 32, 48, 64: the latency tiles, 64 columns
  * wide; 128, 192, 256: the throughput tiles, 128, 256 and 256 wide) and K splits (1-8; at least
- * four K steps of 32 a split on the latency tiles, two on the throughput tiles). With bm = 0 the
- * 256-wide tiles are also run 160 or 224 rows high where that fills the GPU's rounds better. */
+ * four K steps of 32 a split on the latency tiles, two on the throughput tiles). bm = 0: the
+ * library's pick (julia_hip_gemm_pick). */
 typedef struct {
     int bm;
     int splits;
@@ -144,7 +144,8 @@ julia_hip_scratch *julia_hip_scratch_new(size_t ws_floats, size_t counters, char
                                          size_t err_len);
 void julia_hip_scratch_free(julia_hip_scratch *s);
 
-/* src/gemm.rs:254-392 `gemm::launch`: checks, then launches. cfg.bm == 0: the chooser's pick. */
+/* src/gemm.rs:254-392 `gemm::launch`: checks, then launches. cfg.bm == 0: what
+ * julia_hip_gemm_pick says, tiles of any height the library has. */
 int julia_hip_gemm(const julia_hip_gemm_args *g, julia_hip_gemm_config cfg,
                    const julia_hip_scratch *s, void *stream, char *err, size_t err_len);
 
@@ -236,9 +237,17 @@ void julia_hip_synth(uint64_t seed, uint32_t id, uint64_t start, uint64_t count,
 /* f32 -> f16 bits, round to nearest even. */
 void julia_hip_round_f16(const float *in, uint16_t *out, size_t n);
 
-/* This library's tile and split-K chooser for a 256-CU GPU (replaces src/gemm.rs:153-163);
- * epi: the epilogue flags (the throughput tiles take LayerNorm epilogues up to k = 1024). */
+/* This library's tile and split-K chooser for a 256-CU GPU (replaces src/gemm.rs:153-163) among
+ * the tilings that have a name in julia_hip_gemm_config; epi: the epilogue flags (the throughput
+ * tiles take LayerNorm epilogues up to k = 1024). bm = 0 runs heights without a name too, and
+ * other tiles than this choice where those are faster: a caller who does not need a named tiling
+ * passes bm = 0 instead of it. */
 julia_hip_gemm_config julia_hip_gemm_choose(int m, int n, int k, int cus, int epi);
+/* What bm = 0 runs an m x n x k GEMM on, on a GPU of `cus` CUs: the named tiling whose checks
+ * (julia_hip_gemm_check) it passes, and in kernel (nullable, kernel_len bytes, NUL-terminated)
+ * the kernel instance, e.g. "gemm_wide<160, 9, false>". */
+julia_hip_gemm_config julia_hip_gemm_pick(int m, int n, int k, int cus, int epi, char *kernel,
+                                          size_t kernel_len);
 /* The launcher's precondition checks alone (src/gemm.rs:262-329), on the host: 0, or -1 and the
  * reason. The pointers are checked for null and alignment only; the scratch is described by its
  * sizes. */
@@ -288,8 +297,8 @@ const void *julia_hip_engine_tensor(const Engine *e, const char *name, int index
  * on m rows, timed as julia_hip_time_gemm does, rotating through the layers' weights from call
  * to call so they are not L2-resident (src/main.rs:307-312). step: 0 qkv, 1 attention (the
  * layers' own global/window mix), 2 wo, 3 wi, 4 wo_mlp, 5 global attention; the row kernels:
- * 6 embed (m ids), 7 norm_add (m rows), 8 score (every one of m rows). bm = 0: the chooser's
- * tiling. */
+ * 6 embed (m ids), 7 norm_add (m rows), 8 score (every one of m rows). bm = 0: the library's
+ * pick. */
 int julia_hip_time_encoder_step(const Engine *e, int step, int m, int bm, int splits, int warmup,
                                 int batches, int per_batch, float *min_us, float *median_us,
                                 char *err, size_t err_len);

@@ -1045,6 +1045,16 @@ julia_hip_gemm_config julia_hip_gemm_choose(int m, int n, int k, int cus, int ep
     return julia_hip_gemm_config{c.bm, c.splits};
 }
 
+julia_hip_gemm_config julia_hip_gemm_pick(int m, int n, int k, int cus, int epi, char* kernel, size_t kernel_len) {
+    const GemmConfig c = gemm_pick(m, n, k, cus, epi);
+    try {
+        report(kernel, kernel_len, gemm_kernel_name(m, n, k, epi, c, cus > 0 ? cus : 256));
+    } catch (...) {
+        report(kernel, kernel_len, "");
+    }
+    return julia_hip_gemm_config{c.bm, c.splits};
+}
+
 int julia_hip_gemm_check(const julia_hip_gemm_args* g, julia_hip_gemm_config cfg,
                          size_t ws_floats, size_t counters, char* err, size_t err_len) {
     return guarded(err, err_len, [&] {

@@ -207,28 +207,58 @@ static void launch_lat1(const GemmParams& p, int blocks, hipStream_t st) {
     hipLaunchKernelGGL((gemm_lat1<BM, EPI>), dim3(blocks), dim3(512), LDS, st, p);
 }
 
+// The kernel a tiling runs on, on a GPU of `cus` CUs: with a height the one gemm_pick chose, by name the
+// grouped latency kernel and gemm_lat1 (eight waves with a K step each: K >= 256) where the grid is at
+// most a block a CU.
+enum class Kernel { Half, Group, Group2, Lat1, Lat, Big, Wide };
+static Kernel kernel_of(int m, int n, int k, int epi, GemmConfig cfg, int cus) {
+    const int bm = cfg.height ? cfg.height : cfg.bm;
+    if (cfg.bm > 128) return Kernel::Wide;
+    if (cfg.bm == 128) return cfg.height ? Kernel::Group2 : Kernel::Big;
+    if (cfg.splits > 1) return Kernel::Lat;
+    const bool one = (long)(n / 64) * (((long)m + bm - 1) / bm) <= cus;  // a block a CU at most
+    if (gemm_group_takes(bm, k) && (cfg.height || one))
+        return bm == 16 && gemm_group0_takes(m, n, k, cus, epi) ? Kernel::Half : Kernel::Group;
+    return one && k >= 256 ? Kernel::Lat1 : Kernel::Lat;
+}
+
+std::string gemm_kernel_name(int m, int n, int k, int epi, GemmConfig cfg, int cus) {
+    const std::string bm = std::to_string(cfg.height ? cfg.height : cfg.bm), e = std::to_string(epi);
+    const std::string group = "gemm_group<" + bm + ", " + e + ", " + std::to_string(gemm_group_instance(k)) + ", ";
+    const char* split = cfg.splits > 1 ? ", true>" : ", false>";
+    switch (kernel_of(m, n, k, epi, cfg, cus)) {
+        case Kernel::Half: return group + "0>";
+        case Kernel::Group: return group + "1>";
+        case Kernel::Group2: return group + "2>";
+        case Kernel::Lat1: return "gemm_lat1<" + bm + ", " + e + ">";
+        case Kernel::Lat: return "gemm_lat<" + bm + ", " + e + ">";
+        case Kernel::Big: return "gemm_big<" + e + split;
+        default: return "gemm_wide<" + bm + ", " + e + split;
+    }
+}
+
 template <int BM, int EPI>
-static void launch_lat(const GemmParams& p, hipStream_t st) {
+static void launch_lat(const GemmParams& p, bool one, hipStream_t st) {
     const int blocks = p.tiles_n * p.tiles_m * p.splits;
-    // (Eight waves with a K step each: K >= 256.)
-    if (p.splits == 1 && blocks <= device_cus() && p.k >= 256) launch_lat1<BM, EPI>(p, blocks, st);
+    if (one) launch_lat1<BM, EPI>(p, blocks, st);
     else hipLaunchKernelGGL((gemm_lat<BM, EPI>), dim3(blocks), dim3(256), 0, st, p);
 }
 
 // The epilogues only the latency tiles take (the score, gathered rows).
 template <int EPI>
-static void launch_epi_lat(const GemmParams& p, int bm, hipStream_t st) {
+static void launch_epi_lat(const GemmParams& p, Kernel kernel, int bm, hipStream_t st) {
+    const bool one = kernel == Kernel::Lat1;
     switch (bm) {
-        case 16: launch_lat<16, EPI>(p, st); break;
-        case 32: launch_lat<32, EPI>(p, st); break;
-        case 48: launch_lat<48, EPI>(p, st); break;
-        default: launch_lat<64, EPI>(p, st); break;
+        case 16: launch_lat<16, EPI>(p, one, st); break;
+        case 32: launch_lat<32, EPI>(p, one, st); break;
+        case 48: launch_lat<48, EPI>(p, one, st); break;
+        default: launch_lat<64, EPI>(p, one, st); break;
     }
 }
 
 template <int EPI>
-static void launch_epi(const GemmParams& p, int bm, hipStream_t st) {
-    if (bm < 128) return launch_epi_lat<EPI>(p, bm, st);
+static void launch_epi(const GemmParams& p, Kernel kernel, int bm, hipStream_t st) {
+    if (bm < 128) return launch_epi_lat<EPI>(p, kernel, bm, st);
     if (bm > 128) return gemm_wide_launch(p, EPI, bm, st);
     if (p.splits > 1) launch_big<EPI, true>(p, st);
     else launch_big<EPI, false>(p, st);
@@ -249,30 +279,29 @@ void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t st
     p.tiles_n = g.n / (cfg.bm >= 128 ? big_bn(cfg.bm) : 64);
     const int bm = cfg.height ? cfg.height : cfg.bm;
     p.tiles_m = (g.m + bm - 1) / bm;
-    const bool group = cfg.bm < 128 && cfg.splits == 1 && gemm_group_takes(bm, g.k) &&
-                       (cfg.height || p.tiles_n * p.tiles_m <= device_cus());
-    if (group && bm == 16 && gemm_group0_takes(g.m, g.n, g.k, device_cus(), g.epi)) {
+    const Kernel kernel = kernel_of(g.m, g.n, g.k, g.epi, cfg, device_cus());
+    if (kernel == Kernel::Half) {
         p.tiles_n = g.n / 32;
         gemm_group0_launch(p, g.epi, st);
-    } else if (group) gemm_group_launch(p, g.epi, bm, st);
-    else if (cfg.bm == 128 && cfg.height) gemm_group2_launch(p, g.epi, bm, st);
+    } else if (kernel == Kernel::Group) gemm_group_launch(p, g.epi, bm, st);
+    else if (kernel == Kernel::Group2) gemm_group2_launch(p, g.epi, bm, st);
     else switch (g.epi) {
-        case EPI_K_ROPE: launch_epi<EPI_K_ROPE>(p, bm, st); break;
-        case EPI_K_LNROPE: launch_epi<EPI_K_LNROPE>(p, bm, st); break;
-        case EPI_K_LNGEGLU: launch_epi<EPI_K_LNGEGLU>(p, bm, st); break;
-        case EPI_K_RESSTATS: launch_epi<EPI_K_RESSTATS>(p, bm, st); break;
-        case EPI_K_LNBIAS: launch_epi<EPI_K_LNBIAS>(p, bm, st); break;
-        case EPI_K_LNBIASRELU: launch_epi<EPI_K_LNBIASRELU>(p, bm, st); break;
-        case EPI_K_LNBIASGELU: launch_epi<EPI_K_LNBIASGELU>(p, bm, st); break;
-        case EPI_K_BIASRESSTATS: launch_epi<EPI_K_BIASRESSTATS>(p, bm, st); break;
+        case EPI_K_ROPE: launch_epi<EPI_K_ROPE>(p, kernel, bm, st); break;
+        case EPI_K_LNROPE: launch_epi<EPI_K_LNROPE>(p, kernel, bm, st); break;
+        case EPI_K_LNGEGLU: launch_epi<EPI_K_LNGEGLU>(p, kernel, bm, st); break;
+        case EPI_K_RESSTATS: launch_epi<EPI_K_RESSTATS>(p, kernel, bm, st); break;
+        case EPI_K_LNBIAS: launch_epi<EPI_K_LNBIAS>(p, kernel, bm, st); break;
+        case EPI_K_LNBIASRELU: launch_epi<EPI_K_LNBIASRELU>(p, kernel, bm, st); break;
+        case EPI_K_LNBIASGELU: launch_epi<EPI_K_LNBIASGELU>(p, kernel, bm, st); break;
+        case EPI_K_BIASRESSTATS: launch_epi<EPI_K_BIASRESSTATS>(p, kernel, bm, st); break;
         case EPI_K_BIASRESSTATS | EPI_GATHER:
-            launch_epi_lat<EPI_K_BIASRESSTATS | EPI_GATHER>(p, bm, st);
+            launch_epi_lat<EPI_K_BIASRESSTATS | EPI_GATHER>(p, kernel, bm, st);
             break;
-        case EPI_K_LNBIASGELU_SCORE: launch_epi_lat<EPI_K_LNBIASGELU_SCORE>(p, bm, st); break;
+        case EPI_K_LNBIASGELU_SCORE: launch_epi_lat<EPI_K_LNBIASGELU_SCORE>(p, kernel, bm, st); break;
         case EPI_K_LNBIASGELU_SCORE | EPI_GATHER:
-            launch_epi_lat<EPI_K_LNBIASGELU_SCORE | EPI_GATHER>(p, bm, st);
+            launch_epi_lat<EPI_K_LNBIASGELU_SCORE | EPI_GATHER>(p, kernel, bm, st);
             break;
-        case 0: launch_epi<0>(p, bm, st); break;
+        case 0: launch_epi<0>(p, kernel, bm, st); break;
         default: throw std::runtime_error("gemm: no kernel for epilogue " + std::to_string(g.epi));
     }
     const hipError_t e = hipGetLastError();

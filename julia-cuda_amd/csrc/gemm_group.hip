@@ -7,6 +7,8 @@ bool gemm_group_takes(int bm, int k) {
     return k >= 256 && bm <= group_rows_max(group_lines(k)) && group_lds_bytes(bm, k) <= GROUP_LDS_MAX;
 }
 
+int gemm_group_instance(int k) { return group_lines(k); }
+
 // The smallest tile height whose grid is at most a block a CU (0: none). A CU's intake sets the time,
 // so the shortest tiles win wherever they fit (wo at 293 rows: 16-row tiles 3.86 us, 32 4.21, 48
 // 4.80, 64 5.30; wo_mlp 4.46, 5.02, 5.90, 6.62), and the tallest that fit still beat two latency tiles

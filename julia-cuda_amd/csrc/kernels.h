@@ -8,6 +8,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <string>
+
 // f16 storage as its bit pattern in every interface (the device code views it as _Float16),
 // so the host-only and the HIP translation units agree on the types.
 typedef uint16_t jh_half;
@@ -141,6 +143,7 @@ int wide_height(int m, int n, int cus);
 // The grouped latency kernel: whether it takes tiles of bm rows at this k, the height it runs an
 // unsplit m x n x k GEMM with on `cus` CUs (0: it does not), and the launch of a checked GEMM.
 bool gemm_group_takes(int bm, int k);
+int gemm_group_instance(int k);  // its instance that runs k (the K lines of its widest group)
 int gemm_group_height(int m, int n, int k, int cus);
 void gemm_group_launch(const GemmParams& p, int epi, int bm, hipStream_t stream);
 // The same on tiles of 16 rows x 32 columns.
@@ -160,6 +163,8 @@ constexpr int GEMM_BIG_LN_MAX_K = 1024;
 // What a GEMM is run with: the grouped latency kernel or a throughput tile, with its height, in
 // place of gemm_choose's pick.
 GemmConfig gemm_pick(int m, int n, int k, int cus, int epi = 0);
+// The kernel instance that gemm_launch runs a tiling on, on a GPU of `cus` CUs ("gemm_wide<160, 9, false>").
+std::string gemm_kernel_name(int m, int n, int k, int epi, GemmConfig cfg, int cus);
 // Compute units of the current device (queried once per device; 256 if the query fails).
 int device_cus();
 size_t gemm_ws_floats(int m, int n, GemmConfig cfg);

@@ -89,8 +89,8 @@ EXPORTS = [
     "julia_hip_prep_fold_layernorm", "julia_hip_prep_fold_layernorm_bias",
     "julia_hip_prep_geglu_rows", "julia_hip_prep_pack_frag", "julia_hip_prep_unpack_frag",
     "julia_hip_prep_rope_table", "julia_hip_synth",
-    "julia_hip_round_f16", "julia_hip_gemm_choose", "julia_hip_gemm_check", "julia_hip_gemm_plan_2080ti",
-    "julia_hip_gemm_choose_2080ti", "julia_hip_engine_info_get", "julia_hip_engine_tensor",
+    "julia_hip_round_f16", "julia_hip_gemm_choose", "julia_hip_gemm_pick", "julia_hip_gemm_check",
+    "julia_hip_gemm_plan_2080ti", "julia_hip_gemm_choose_2080ti", "julia_hip_engine_info_get", "julia_hip_engine_tensor",
     "julia_hip_time_encoder_step", "julia_hip_profile_layer", "julia_hip_run_trace",
     "julia_hip_encode_batch",
     "julia_hip_encode_batch_phases", "julia_hip_checkpoint_config", "julia_hip_answer",
@@ -154,6 +154,7 @@ def lib():
                                   _CP, _SZ]),
         "julia_hip_latency_summary": (_I, [_F64P, _SZ, _F64P]),
         "julia_hip_gemm_choose": (GemmConfig, [_I, _I, _I, _I, _I]),
+        "julia_hip_gemm_pick": (GemmConfig, [_I, _I, _I, _I, _I, _CP, _SZ]),
         "julia_hip_gemm_check": (_I, [ctypes.POINTER(GemmArgs), GemmConfig, _SZ, _SZ, _CP, _SZ]),
         "julia_hip_gemm_plan_2080ti": (None, [_I, _I, _I, _I, _I, ctypes.POINTER(_I),
                                               ctypes.POINTER(_I)]),
@@ -586,6 +587,15 @@ def gemm_choose(m, n, k, cus=256, epi=0):
         epi = EPI[epi]
     c = lib().julia_hip_gemm_choose(m, n, k, cus, epi)
     return c.bm, c.splits
+
+
+def gemm_pick(m, n, k, cus=256, epi=0):
+    """What bm = 0 runs: (bm, splits) of the named tiling whose checks it passes, the kernel instance."""
+    if isinstance(epi, str):
+        epi = EPI[epi]
+    name = ctypes.create_string_buffer(64)
+    c = lib().julia_hip_gemm_pick(m, n, k, cus, epi, name, 64)
+    return c.bm, c.splits, name.value.decode()
 
 
 def gemm_check(args, bm, splits=1, ws_floats=0, counters=0):

@@ -258,7 +258,7 @@ def test_chooser_at_row_edges(torch_cuda, scratch, kind, n, k):
     for m in (1, 15, 17, 47, 49, 255, 257, 1023, 2049):
         P = gemm_problem(kind, m, n, k, seed=500 + m + n)
         out, st = run_gemm(torch_cuda, P, 0, 1, scratch)
-        check_gemm(P, out, st, f"{kind} m={m} chosen {tuple(jh.gemm_choose(m, n, k, 256, P['epi']))}")
+        check_gemm(P, out, st, f"{kind} m={m} runs {jh.gemm_pick(m, n, k, 256, P['epi'])[2]}")
 
 
 # K split on the throughput tiles: the last arriver's sum in split order, then every kind of

@@ -255,11 +255,35 @@ def _model_gemms(d, inter=1152, ff=1536):
             (d, ff, "biasresstats"), (d, d, "lnbiasgelu")]
 
 
+def check_kernel(kernel, m, n, k, flags, cus=256):
+    """A picked kernel instance holds its tile: heights, columns, LDS, and a block a CU where it
+    takes a CU for itself."""
+    name, args = re.match(r"(\w+)<(.*)>$", kernel).groups()
+    args = args.replace("false", "0").split(", ")
+    rows = 128 if name == "gemm_big" else int(args[0])
+    assert int(args[0 if name == "gemm_big" else 1]) == flags, kernel
+    if name == "gemm_group":
+        lines, half = int(args[2]), int(args[3])
+        assert 256 <= k <= 1536 and lines == max(2, -(-k // 256)), (kernel, k)
+        assert rows * k * 2 <= 160 * 1024 and 4 * rows * 68 * 4 + 16 <= 160 * 1024, (kernel, k)
+        cols = (32, 64, 128)[half]
+        assert n % cols == 0 and n // cols * -(-m // rows) <= cus, (kernel, m, n)
+        assert not (cols == 32 and (rows != 16 or flags & jh.EPI_STATS)), kernel
+    elif name in ("gemm_lat", "gemm_lat1"):
+        assert rows in (16, 32, 48, 64), kernel
+        assert (name == "gemm_lat1") == (n // 64 * -(-m // rows) <= cus and k >= 256), (kernel, m, n, k)
+    elif name == "gemm_wide":
+        assert rows in (160, 192, 224, 256) and n % 256 == 0 and args[2] == "0", (kernel, n)
+    else:
+        assert name == "gemm_big" and n % 128 == 0 and args[1] == "0", (kernel, n)
+
+
 @pytest.mark.parametrize("d", [384, 768, 1280, 2048])
 def test_every_pick_passes_the_launch_checks(d):
-    """gemm_choose's pick for every model GEMM (with its epilogue) at every row count passes the
-    launcher's own precondition checks (src/gemm.rs:262-329): in particular the throughput tiles'
-    LayerNorm limit (k <= 1024), which widths past 1024 reach."""
+    """gemm_choose's named tiling and gemm_pick's, what bm = 0 runs, for every model GEMM (with its
+    epilogue) at every row count pass the launcher's own precondition checks (src/gemm.rs:262-329):
+    in particular the throughput tiles' LayerNorm limit (k <= 1024), which widths past 1024 reach.
+    gemm_pick takes no K split, so no scratch, and its kernel holds the tile."""
     base = 1 << 20  # 16-byte aligned stand-in addresses (the check does not dereference them)
     for m in list(range(1, 4097, 37)) + [8192, 18752, 20000]:
         for n, k, epi in _model_gemms(d):
@@ -276,8 +300,11 @@ def test_every_pick_passes_the_launch_checks(d):
             args = jh.gemm_args(flags, base, base + 4096, base + 8192, m, n, k, **kw)
             bm, sp = jh.gemm_choose(m, n, k, 256, flags)
             jh.gemm_check(args, bm, sp, ws_floats=1 << 30, counters=1 << 20)
+            pick, split, kernel = jh.gemm_pick(m, n, k, 256, flags)
+            jh.gemm_check(args, pick, split)
+            check_kernel(kernel, m, n, k, flags)
             if flags & jh.EPI_LN and k > 1024:
-                assert bm < 128, (m, n, k, epi, bm)
+                assert bm < 128 and pick < 128, (m, n, k, epi, bm)
 
 
 def test_gemm_check_rejects_what_the_kernels_do_not_take():
