@@ -380,6 +380,19 @@ void gemm_launch_static(const Gemm& g, GemmConfig cfg, hipStream_t st) {
     gemm_launch(g, cfg, s, st);
 }
 
+// The cheapest latency tile and its time (us; the model below).
+static GemmConfig latency_choose(int m, int n, int k, int cus, double& us) {
+    GemmConfig best{32, 1};
+    us = 1e30;
+    for (int bm : {16, 32, 48, 64}) {
+        const long tiles = (long)(n / 64) * (((long)m + bm - 1) / bm);
+        const long per_cu = (tiles + cus - 1) / cus;
+        const double cost = 4.0 + (double)per_cu * (bm + 64) * k * 2 / 55e3;
+        if (cost < us - 0.05) us = cost, best = GemmConfig{bm, 1};
+    }
+    return best;
+}
+
 // The tiling for a GEMM on a 256-CU GPU, by name (julia_hip_gemm_choose): the cheapest of the
 // latency tiles and the three throughput tiles under a cost model fitted to MI355X sweeps (M = 72 .. 18752, the encoder's
 // four shapes; microseconds, random operands, weights rotating through the layers).
@@ -405,14 +418,8 @@ GemmConfig gemm_choose(int m, int n, int k, int cus, int epi) {
     static_assert(GEMM_BIG_LN_MAX_K == 128 * BIG_LN_SLOTS && GEMM_BIG_LN_MAX_K == 128 * WIDE_LN_SLOTS,
                   "the LayerNorm limit of the throughput tiles");
     if (cus <= 0) cus = 256;
-    GemmConfig best{32, 1};
     double best_cost = 1e30;
-    for (int bm : {16, 32, 48, 64}) {
-        const long tiles = (long)(n / 64) * ((m + bm - 1) / bm);
-        const long per_cu = (tiles + cus - 1) / cus;
-        const double cost = 4.0 + (double)per_cu * (bm + 64) * k * 2 / 55e3;
-        if (cost < best_cost - 0.05) best_cost = cost, best = GemmConfig{bm, 1};
-    }
+    GemmConfig best = latency_choose(m, n, k, cus, best_cost);
     if (m >= 640 && n % 128 == 0 && k % 64 == 0 && !((epi & EPI_LN) && k > GEMM_BIG_LN_MAX_K)) {
         const double ks = (double)k / 768.0;
         const long l128 = ((long)(n / 128) * ((m + 127) / 128) + cus - 1) / cus;
@@ -430,34 +437,49 @@ GemmConfig gemm_choose(int m, int n, int k, int cus, int epi) {
     return best;
 }
 
-// What a GEMM is run with: gemm_choose's pick, a throughput one decided between the 128 x 128 and the
-// wide tiles at their best height by a model of the kernels as they are (MI355X, random operands):
-//  - 128 x 128 tiles (two a CU): ~2 us plus ~8.5 us (K = 768) for one a CU, ~2.5 us plus 7.6 us
-//    each for more (measured 10.7 us for one, 15-17.5 for two, 25 for three, 39 for five).
-//  - The wide tiles (one a CU): ~4.5 us plus, per round of tiles, the K loop (3.2 + h / 20 us at K =
-//    768, h the tile's rows) and the epilogue (0.2 + h / 80): measured at 160 rows 18.5 us for one
-//    round (4096 x 2304), 33.7 for two (8192), at 224 rows 66 for three (18752).
-// So 128 x 128 for qkv and wi up to ~3000 rows and for wo up to 8192 (17.5 us there against 18.5
-// for the wide tiles; wo_mlp level, 23.5), the wide tiles for qkv and wi from 4096 (18.5 us
-// against 25) and for everything at 18752.
-// And before these, wherever a grid of at most a block a CU covers the GEMM, the grouped latency
-// kernel at its smallest such height, on 64 columns or else on 128 (gemm_group.hip and gemm_group2.hip
-// have the figures).
+// What a GEMM is run with (bm = 0), a model of the kernels as they are, us, random operands, weights
+// not in L2 (MI355X):
+//  - wherever a grid of at most a block a CU covers the GEMM, the grouped latency kernel at its smallest
+//    such height, on 64 columns or else on 128 (gemm_group.hip and gemm_group2.hip have the figures);
+//  - else, below 640 rows and where a throughput tile does not take the GEMM, gemm_choose's latency tile;
+//  - else the least of that where its grid is at most a block a CU (two on a CU were never faster than
+//    128 x 128 tiles: wo, wo_mlp and linear2, K = 1536, at 5384 rows 22.1, 32, 39 us against 15.6, 19.2,
+//    26.1, linear2 at 2300 rows 20.7 against 17.1), the 128 x 128 and the wide tiles at their best height
+//    (wide_height).
+// ks: K / 768; x: 128 x 128 tiles a CU, two at a time. One a CU: 2 + 8.5 ks up to K = 614, 3.6 + 6.5 ks
+// past it (measured 7.0-7.9 at K = 384, 9.9-10.9 at 768, 12.5-14.4 at 1152, 16-18 at 1536, 25 at 2560).
+// Two: 5.4 + 11.4 ks, 8% less while hardly a CU has a second one, 4% more per tenth from x = 1.7 on
+// (768 columns, 5448 / 8192 / 10500 rows: K = 768 15.5 / 17.0 / 18.9, K = 1152 19.0 / 22.0 / 24.7, K =
+// 1536 26.0 / 28.4 / 32.4). More: 1.5 + 1.9 and 6.1 ks a tile (three 25.3, 33.8, 43.3 at those K).
+// The wide tiles (one a CU): 4.8 us, and a round of tiles h high 0.5 + h / 80 + ks (2.9 + 0.046 h). Where
+// most CUs have a tile, all ask for the residual and store at the same time: 5.5 us times the share of
+// them past 0.42; GELU 2.5, GeGLU 0.8 (K = 1152, 160 rows: 5448 rows 22.2, 8192 23.1, 10500 24.5).
+// The line between the two at wo_mlp's K = 1152: 128 x 128 up to 10496 rows (8192 rows 22.1 against 23.1,
+// 5448 rows 19.0 against 22.2), at K = 768 up to 10880 (two tiles a CU); for qkv 3200 (3300 rows
+// 17.0 against 16.1), for wi 3456 (3300 rows 18.1 against 18.5).
 GemmConfig gemm_pick(int m, int n, int k, int cus, int epi) {
     if (cus <= 0) cus = 256;
     if (const int h = gemm_group_height(m, n, k, cus)) return GemmConfig{std::min(h, 64), 1, h};
     if (const int h = gemm_group2_height(m, n, k, cus, epi)) return GemmConfig{128, 1, h};
-    GemmConfig best = gemm_choose(m, n, k, cus, epi);
-    if (best.bm < 128) return best;
+    double best_cost = 0.0;
+    GemmConfig best = latency_choose(m, n, k, cus, best_cost);
+    if (m < 640 || n % 128 || k % 64 || ((epi & EPI_LN) && k > GEMM_BIG_LN_MAX_K)) return best;
+    if ((long)(n / 64) * (((long)m + best.bm - 1) / best.bm) > cus) best_cost = 1e30;
     const double ks = (double)k / 768.0;
-    const long l128 = ((long)(n / 128) * ((m + 127) / 128) + cus - 1) / cus;
-    best = GemmConfig{128, 1};
+    const double x = (double)(n / 128) * (double)(((long)m + 127) / 128) / cus;
+    const double c128 = x <= 1.0   ? std::min(2.0 + 8.5 * ks, 3.6 + 6.5 * ks)
+                        : x <= 2.0 ? (5.4 + 11.4 * ks) * (x <= 1.04 ? 0.92 : 1.0 + std::max(0.0, 0.4 * (x - 1.7)))
+                                   : 1.5 + std::ceil(x) * (1.9 + 6.1 * ks);
+    if (c128 < best_cost) best_cost = c128, best = GemmConfig{128, 1};
     if (n % WIDE_BN == 0) {
         const int h = wide_height(m, n, cus);
-        const long rounds = ((long)(n / WIDE_BN) * ((m + h - 1) / h) + cus - 1) / cus;
-        const double c128 = l128 == 1 ? 2.0 + 8.5 * ks : 2.5 + 7.6 * ks * (double)l128;
-        if (4.5 + (double)rounds * (0.2 + h / 80.0 + ks * (3.2 + h / 20.0)) < c128)
-            best = GemmConfig{256, 1, h};
+        const double tiles = (double)(n / WIDE_BN) * (double)(((long)m + h - 1) / h);
+        const double rounds = std::ceil(tiles / cus), share = tiles / (rounds * cus);
+        double round = 0.5 + h / 80.0 + ks * (2.9 + 0.046 * h);
+        if (epi & EPI_RES) round += 5.5 * std::max(0.0, share - 0.42);
+        if (epi & EPI_GELU) round += 2.5;
+        if (epi & EPI_GEGLU) round += 0.8;
+        if (4.8 + rounds * round < best_cost) best = GemmConfig{256, 1, h};
     }
     return best;
 }

@@ -307,6 +307,22 @@ def test_every_pick_passes_the_launch_checks(d):
                 assert bm < 128 and pick < 128, (m, n, k, epi, bm)
 
 
+@pytest.mark.parametrize("n,k,epi,picks", [
+    (768, 768, "resstats", {2688: "gemm_group<64", 3000: "gemm_big", 5384: "gemm_big", 8192: "gemm_big", 12000: "gemm_wide"}),
+    (768, 1152, "resstats", {5384: "gemm_big", 5448: "gemm_big", 8192: "gemm_big", 11000: "gemm_wide<160", 18752: "gemm_wide<224"}),
+    (768, 1536, "biasresstats", {2016: "gemm_group", 2300: "gemm_big", 5447: "gemm_big", 5774: "gemm_wide", 12000: "gemm_wide"}),
+    (2304, 768, "lnrope", {800: "gemm_group", 1024: "gemm_big", 3000: "gemm_big", 4096: "gemm_wide<160", 18752: "gemm_wide<224"}),
+    (768, 768, "lnbiasgelu", {6: "gemm_group<16", 8192: "gemm_big", 10500: "gemm_big", 11000: "gemm_wide"}),
+    (3072, 1024, "lngeglu", {1500: "gemm_big", 2035: "gemm_big", 5000: "gemm_wide"}),
+    (768, 128, "lnbiasrelu", {5774: "gemm_big", 12000: "gemm_wide"}),
+    (768, 2048, "resstats", {700: "gemm_lat1", 3000: "gemm_big"})])
+def test_pick_matches_the_measured_winners(n, k, epi, picks):
+    """What bm = 0 runs at sizes on both sides of the kernels' crossings on 256 CUs, the fastest of
+    them there by a margin (MI355X, weights not in L2; the figures stand with gemm_pick)."""
+    for m, kernel in picks.items():
+        assert jh.gemm_pick(m, n, k, 256, epi)[2].startswith(kernel), (m, jh.gemm_pick(m, n, k, 256, epi))
+
+
 def test_gemm_check_rejects_what_the_kernels_do_not_take():
     base = 1 << 20
     ln = dict(stats_in=base + 64, colsum=base + 128)
