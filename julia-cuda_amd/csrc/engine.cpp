@@ -327,9 +327,12 @@ struct Engine {
         // With fewer markers than rows the head's last steps run on the marker rows alone. The
         // GEMM that first reads them gathers them itself (EPI_GATHER: out_proj of the last head
         // layer, or the scorer's lin1 without head layers), and the score rides on lin1's
-        // epilogue (EPI_SCORE), where the chooser gives those GEMMs latency tiles (lin1 without
-        // a K split); otherwise a gather kernel and a score kernel run.
-        auto lat = [&](GemmConfig c) { return c.bm < 128; };
+        // epilogue (EPI_SCORE), where those GEMMs run on latency tiles of up to 64 rows (lin1
+        // without a K split); otherwise a gather kernel and a score kernel run. (Past them, 2688
+        // marker rows at d = 384 and 1344 at 768, the score's sum by one block grows past what the
+        // two launches cost: from 2400 to 4000 of 16000 rows at d = 384 a pass takes 11 us more
+        // folded, 8.5 with the two kernels.)
+        auto lat = [&](GemmConfig c) { return c.bm < 128 && c.height <= 64; };
         const GemmConfig cs = compact ? gemm_pick(nm, d, d, cus, EPI_K_LNBIASGELU) : GemmConfig{};
         const bool fold = compact && lat(cs) && cs.splits == 1 &&
                           (L == 0 || lat(gemm_pick(nm, d, d, cus, EPI_K_BIASRESSTATS)));

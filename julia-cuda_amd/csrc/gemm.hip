@@ -145,6 +145,7 @@ void gemm_check(const Gemm& g, GemmConfig cfg, const Scratch& s) {
     const bool gather = g.epi & EPI_GATHER, score = g.epi & EPI_SCORE;
     if (gather != (g.rows != nullptr) || (gather && (tput || g.src_m < 1)))
         fail("gathered rows go with the gather epilogues on the latency tiles, from src_m >= 1 rows");
+    if ((gather || score) && cfg.height > 64) fail("gathered rows and the score take tiles of up to 64 rows");
     if (gather && (g.epi & EPI_RES) && !g.res) fail("gathered rows need a separate residual");
     if (score != (g.score_w != nullptr && g.logits != nullptr))
         fail("score weights and logits go with the score epilogue");

@@ -226,14 +226,19 @@ void launch_group_lines(const GemmParams& p, hipStream_t st) {
 template <int EPI>
 void launch_group_epi(const GemmParams& p, int bm, hipStream_t st) {
     switch (bm) {
-        case 16: launch_group_lines<16, EPI, 1>(p, st); break;
-        case 32: launch_group_lines<32, EPI, 1>(p, st); break;
-        case 48: launch_group_lines<48, EPI, 1>(p, st); break;
-        case 64: launch_group_lines<64, EPI, 1>(p, st); break;
-        case 80: launch_group_lines<80, EPI, 1>(p, st); break;
-        case 96: launch_group_lines<96, EPI, 1>(p, st); break;
-        default: launch_group_lines<128, EPI, 1>(p, st); break;
+        case 16: launch_group_lines<16, EPI, 1>(p, st); return;
+        case 32: launch_group_lines<32, EPI, 1>(p, st); return;
+        case 48: launch_group_lines<48, EPI, 1>(p, st); return;
+        case 64: launch_group_lines<64, EPI, 1>(p, st); return;
     }
+    if constexpr (!(EPI & (EPI_GATHER | EPI_SCORE))) {  // (gathered rows and the score: up to 64 rows)
+        switch (bm) {
+            case 80: launch_group_lines<80, EPI, 1>(p, st); return;
+            case 96: launch_group_lines<96, EPI, 1>(p, st); return;
+            case 128: launch_group_lines<128, EPI, 1>(p, st); return;
+        }
+    }
+    throw std::runtime_error("gemm: no grouped kernel of " + std::to_string(bm) + " rows");
 }
 
 template <int EPI>
