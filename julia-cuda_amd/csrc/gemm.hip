@@ -1,17 +1,18 @@
 // The fused-epilogue GEMM family on MFMA (gfx950): c = epilogue(a . w^T), f16 in, f32
 // accumulate, f16 out. The reference's tensor-core GEMM (kernels/src/gemm.rs, gemm_tile in
 // kernels/src/main.rs:886-1041) walks K through shared tiles with 4-8 warps each owning a
-// piece of the output; here two kernels cover the two regimes of a 256-CU GPU:
+// piece of the output; here four kernels cover the regimes of a 256-CU GPU:
 //
-//  - gemm_group (16 to 128 rows x 64 columns, 32 to 64 x 128, 16 x 32,
-//    gemm_group.h): the latency-bound regime, grids of at
-//    most a block a CU (every GEMM of a request of up to 672 tokens): eight waves in four K groups,
-//    a's rows whole in LDS, w straight into registers, the partial tiles summed through LDS.
-//  - gemm_lat (BM = 16/32/48/64 rows x 64 columns): more tiles than CUs, or a K split. The block's
-//    four waves split K between them, streaming a and w fragments from L2 into registers, two
-//    blocks a CU. Grid split-K on top is deterministic: the last block of a tile to arrive sums
-//    every split's partial in split order. gemm_lat1, its eight-wave form on a CU of its own, is
-//    left for the K that gemm_group does not hold (past 1536).
+//  - gemm_group (16 to 128 rows x 64 columns, 32 to 64 x 128, 16 x 32, gemm_group.h): the
+//    latency-bound regime, grids of at most a block a CU (every GEMM of a request of up to 896
+//    tokens): eight waves in four K groups, a's rows whole in LDS, w straight into registers, the
+//    partial tiles summed through LDS.
+//  - gemm_lat (BM = 16/32/48/64 rows x 64 columns): more tiles than CUs of a GEMM that no throughput
+//    tile takes, a tiling by name, or a K split. The block's four waves split K between them,
+//    streaming a and w fragments from L2 into registers, two blocks a CU. Grid split-K on top is
+//    deterministic: the last block of a tile to arrive sums every split's partial in split order.
+//    gemm_lat1, its eight-wave form on a CU of its own, is left for the K that gemm_group does not
+//    hold (past 1536).
 //  - gemm_big (128 x 128 tiles): the middle sizes and widths that 256 does not divide: a and w
 //    tiles copied into four LDS stages by direct buffer -> LDS loads (gemm_big.h), four waves each
 //    owning a 64 x 64 output block on 32 x 32 x 16 MFMA, the epilogue's column-wise part applied on
@@ -21,7 +22,7 @@
 // A K split of the throughput tiles, the same deterministic last-arriver sum, is there for
 // completeness (config sweeps): at these sizes the chooser never picks one.
 //
-// Both apply the epilogues of device.h (LayerNorm folding, bias, ReLU/GELU, RoPE, GeGLU,
+// All apply the epilogues of device.h (LayerNorm folding, bias, ReLU/GELU, RoPE, GeGLU,
 // residual, output statistics) in the same order.
 #include <algorithm>
 #include <mutex>
@@ -395,8 +396,10 @@ static GemmConfig latency_choose(int m, int n, int k, int cus, double& us) {
 }
 
 // The tiling for a GEMM on a 256-CU GPU, by name (julia_hip_gemm_choose): the cheapest of the
-// latency tiles and the three throughput tiles under a cost model fitted to MI355X sweeps (M = 72 .. 18752, the encoder's
-// four shapes; microseconds, random operands, weights rotating through the layers).
+// latency tiles and the three throughput tiles under a cost model fitted to MI355X sweeps (M = 72 ..
+// 18752, the encoder's four shapes; microseconds, random operands, weights rotating through the
+// layers) of the kernels that these names ran before gemm_group and gemm_wide: callers have its
+// choices. What bm = 0 runs is gemm_pick's.
 //  - Latency tiles (BM = 16/32/48/64 x 64): bound by how fast a CU takes in its tiles'
 //    operands: a fixed ~4 us (launch, first round trip, reduction, epilogue) plus the busiest
 //    CU's operand bytes, ceil(tiles / CUs) x (BM + 64) x K x 2, at about 55 GB/s into one CU.

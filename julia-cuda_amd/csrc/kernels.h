@@ -156,12 +156,12 @@ void gemm_group2_launch(const GemmParams& p, int epi, int bm, hipStream_t stream
 // Throws std::runtime_error when g or cfg break what the kernels assume.
 void gemm_check(const Gemm& g, GemmConfig cfg, const Scratch& s);
 void gemm_launch(const Gemm& g, GemmConfig cfg, const Scratch& s, hipStream_t stream);
-// The tile height and split-K for an m x n x k GEMM with epilogue `epi` on `cus` compute units
-// (the throughput tiles only where they take the epilogue: LayerNorm up to k = GEMM_BIG_LN_MAX_K).
+// The tile height and split-K, by name, for an m x n x k GEMM with epilogue `epi` on `cus` compute
+// units (the throughput tiles only where they take the epilogue: LayerNorm up to k =
+// GEMM_BIG_LN_MAX_K).
 GemmConfig gemm_choose(int m, int n, int k, int cus, int epi = 0);
 constexpr int GEMM_BIG_LN_MAX_K = 1024;
-// What a GEMM is run with: the grouped latency kernel or a throughput tile, with its height, in
-// place of gemm_choose's pick.
+// What a GEMM is run with: the fastest of all kernels, with its height where it has one.
 GemmConfig gemm_pick(int m, int n, int k, int cus, int epi = 0);
 // The kernel instance that gemm_launch runs a tiling on, on a GPU of `cus` CUs ("gemm_wide<160, 9, false>").
 std::string gemm_kernel_name(int m, int n, int k, int epi, GemmConfig cfg, int cus);

@@ -6,7 +6,7 @@
 # of every HIP-event figure in the bench line), traffic (FETCH_SIZE / WRITE_SIZE passes of the
 # 293-token roofline kernels, calibrated by the library's copy kernel). The
 # graph-replayed forward pass is not profiled: a run of it under rocprofv3 ended in a host
-# segmentation fault inside a HIP call, its cause not known. Writes raw output under OUT and the
+# segmentation fault inside hipGraphLaunch, its cause not known. Writes raw output under OUT and the
 # summaries bench.py reads under OUT/profiles_new (copy them to profiles/).
 set -o pipefail
 R=$(cd "$(dirname "$0")/.." && pwd)

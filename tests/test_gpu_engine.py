@@ -253,7 +253,7 @@ def test_batched_encoder_matches_each_request(torch_cuda):
 
 
 def test_batched_encoder_on_256_tiles(torch_cuda):
-    """The persistent kernel's 256 x 256 instance (512-thread blocks, the streaming attention
+    """The persistent kernel's wide instance (256 in the plan, 192-row tiles here; 512-thread blocks, the streaming attention
     tile on eight waves): config 4's widths, a batch past 2048 rows; the layer kernel against
     the per-step kernels."""
     c = dict(d=768, layers=2, inter=1152, vocab=1000, head_ff=768, max_positions=4096, seed=11,
@@ -298,7 +298,7 @@ def test_persistent_kernel_on_either_wide_height(torch_cuda, rows):
 
 
 def test_whole_model_on_256_tiles(torch_cuda):
-    """The whole-model launch on the 256 x 256 instance (config 4's widths, head_ff 1536, a
+    """The whole-model launch on the wide instance (256 in the plan; config 4's widths, head_ff 1536, a
     batched pass past 2048 rows): every head GEMM on the throughput tile, attention bounded to
     each request, every question type; against the per-step kernels on the same pass and the
     oracle on single requests."""
@@ -327,7 +327,7 @@ def test_whole_model_on_256_tiles(torch_cuda):
 
 
 def test_fused_fallback_when_the_head_does_not_fit(torch_cuda):
-    """A head the 256 x 256 instance cannot take (head_ff 1152, not a multiple of 256): the
+    """A head the wide instances cannot take (head_ff 1152, not a multiple of 256): the
     layer_fused pass falls back to the encoder kernel and the head's own launches, and still
     matches the per-step kernels."""
     c = dict(d=768, layers=2, inter=1152, vocab=1000, head_ff=1152, max_positions=4096, seed=13)
